@@ -236,9 +236,9 @@ int vm_hip_qmm_f32_noalloc(const float* a, const int8_t* wq, const float* scale,
  * Same operation for the reference's mixed-precision dtype keys
  * (src/cpu/ops/quantized_matmul.cpp:363-367): (a, scale, c) dtypes in
  * {(F32,F32,F32), (F16,F16,F16), (F16,F32,F16), (BF16,BF16,BF16),
- * (BF16,F32,BF16)}.  Half inputs are widened to fp32, accumulation is fp32
- * and half outputs are rounded to nearest even (include/velomind/dtype.h:
- * 53-107).
+ * (BF16,F32,BF16)}.  16-bit activations are multiplied as they are (by codes
+ * that are exact in the same type), accumulation is fp32 and half outputs
+ * are rounded to nearest even (include/velomind/dtype.h:53-107).
  */
 int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale,
                int scale_dtype, void* c, int c_dtype, int64_t rows_m, int64_t k, int64_t n,
@@ -684,7 +684,7 @@ int vm_hip_gemv_trace_read(void* host, int64_t bytes);
  * counterpart; the resident decoder's prompts) ---------------------------
  * vm_hip_qmm_f32 with more than 4 rows first stages A in a pre-pass: each
  * row scaled by a power of two and split into two fp16 parts (22
- * significant bits), row-major or in the wide MFMA kernel's operand order.
+ * significant bits), row-major or in the MFMA kernel's operand order.
  * A producer that holds whole rows can write that layout itself instead:
  * vm_hip_qmm_a_layout says which layout (VM_HIP_A_FP32: the shape takes
  * fp32 A only, as every row longer than 6144 does, the producers' limit)

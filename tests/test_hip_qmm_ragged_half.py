@@ -1,0 +1,107 @@
+"""The MFMA quantized matmul where its tiles end: K that is no multiple of
+the 32-row chunk, N that is no multiple of a lane's four columns, row counts
+around the 16- and 32-row tiles, and fp16 / bf16 activations and outputs with
+scales of either type, against the product in 64 bits.
+
+fp32 bound: A is split at 22 bits and 2 k products are summed in fp32, so
+|err| <= (2^-22 + 2 k 2^-24) sum |a w|.  16-bit activations are used as they
+are: k products summed in fp32, then one rounding of the output (2^-11 of it
+for fp16, 2^-8 for bf16, half an ulp of 11 and 8 bits, and 2^-24 where fp16 is subnormal)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(rng, kind, block, k, n):
+    """(codes, scales, code values as float64, quant type)"""
+    if kind == "int4":
+        packed, s = O.quantize_int4((rng.standard_normal((k, n)) * 0.02).astype(np.float32), block)
+        v = np.empty((2 * packed.shape[0], n), np.int8)
+        v[0::2] = (packed.view(np.int8) << 4) >> 4
+        v[1::2] = packed.view(np.int8) >> 4
+        return packed, s, v[:k].astype(np.float64), 2
+    if block == 0:
+        q, s = O.quantize_int8((rng.standard_normal((k, n)) * 0.02).astype(np.float32))
+        return q, s.reshape(1, n), q.astype(np.float64), 1
+    q = rng.integers(-127, 128, (k, n), dtype=np.int8)
+    return q, (rng.random((-(-k // block), n)) * 0.01 + 1e-4).astype(np.float32), q.astype(np.float64), 1
+
+
+def _dense(values, scales, block):
+    k = values.shape[0]
+    return values * scales.astype(np.float64).repeat(block or k, 0)[:k]
+
+
+KINDS = [("int8", 0), ("int8", 96), ("int4", 32), ("int4", 64)]
+
+
+@pytest.mark.parametrize("kind,block", KINDS)
+@pytest.mark.parametrize("m,k,n", [(5, 31, 16), (7, 33, 17), (16, 1001, 67), (17, 224, 131), (33, 1, 19), (40, 95, 1027),
+                                   (100, 2047, 515), (129, 64, 130)])
+def test_ragged_fp32(hip, kind, block, m, k, n):
+    rng = np.random.default_rng(m * 1000 + k + n + block)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    print(f"case ragged {kind} block={block} m={m} k={k} n={n}", flush=True)
+    out = hip.run_qmm(x, q, s, k, qt, block).astype(np.float64)
+    wd = _dense(v, s, block)
+    mag = np.abs(x.astype(np.float64)) @ np.abs(wd)
+    assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * mag + 1e-30)
+
+
+def _bits(x, bf16):
+    return O.f32_to_bf16_bits(x) if bf16 else O.f32_to_f16_bits(x)
+
+
+def _wide(bits, bf16):
+    return (bits.astype(np.uint32) << 16).view(np.float32) if bf16 else bits.view(np.float16).astype(np.float32)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("half_scale", [False, True])
+@pytest.mark.parametrize("kind,block", KINDS)
+@pytest.mark.parametrize("m,k,n", [(1, 256, 96), (3, 2048, 515), (4, 33, 20), (16, 992, 336), (31, 224, 67), (70, 320, 258),
+                                   (130, 1000, 132), (200, 2048, 1100)])
+def test_half(hip, bf16, half_scale, kind, block, m, k, n):
+    rng = np.random.default_rng(m + k + n + block)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    # fp16 rows from 1e-7 (subnormal) to 1e3; a bf16 row of 1e30
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x *= np.float32(10.0) ** rng.integers(-3, 4, (m, 1)).astype(np.float32)
+    x[0] *= np.float32(1e30 if bf16 else 1e-6)
+    a = _bits(x, bf16)
+    sb = _bits(s, bf16) if half_scale else s
+    dt = hip.DTYPE_BF16 if bf16 else hip.DTYPE_F16
+    da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (a, q.view(np.int8), sb, np.zeros((m, n), np.uint16)))
+    print(f"case half bf16={bf16} half_scale={half_scale} {kind} block={block} m={m} k={k} n={n}", flush=True)
+    hip.qmm(da.addr, dt, dq.addr, ds.addr, dt if half_scale else hip.DTYPE_F32, dc.addr, dt, m, k, n, qt, block)
+    out = _wide(dc.download(np.uint16, (m, n)), bf16).astype(np.float64)
+    wd = _dense(v, _wide(sb, bf16) if half_scale else s, block)
+    aw = _wide(a, bf16).astype(np.float64)
+    ref, mag = aw @ wd, np.abs(aw) @ np.abs(wd)
+    ulp = 2.0 ** -8 if bf16 else 2.0 ** -11
+    fits = np.abs(ref) < (3e38 if bf16 else 65000)
+    bound = ulp * 1.01 * np.abs(ref) + 2 * k * 2.0 ** -24 * mag + 2.0 ** -24 * (not bf16)
+    assert np.all(np.abs(out - ref)[fits] <= bound[fits]), np.max((np.abs(out - ref) / bound)[fits])
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_half_infinity_and_nan(hip, bf16):
+    # 5 x 64 times 64 x 32 codes that are never zero: a row's infinity reaches
+    # every output of the row, a NaN too, and other rows stay as they were
+    m, k, n = 5, 64, 32
+    rng = np.random.default_rng(3)
+    q = rng.integers(1, 128, (k, n), dtype=np.int8)
+    s = np.ones((1, n), np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1, 7], x[3, 60] = np.inf, np.nan
+    dt = hip.DTYPE_BF16 if bf16 else hip.DTYPE_F16
+    da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (_bits(x, bf16), q, s, np.zeros((m, n), np.uint16)))
+    hip.qmm(da.addr, dt, dq.addr, ds.addr, hip.DTYPE_F32, dc.addr, dt, m, k, n, 1, 0)
+    out = _wide(dc.download(np.uint16, (m, n)), bf16)
+    assert np.all(np.isposinf(out[1])) and np.all(np.isnan(out[3])) and np.all(np.isfinite(out[[0, 2, 4]]))

@@ -58,10 +58,9 @@ def _run(cmd: list[str]) -> None:
             sys.stderr.write(line + "\n")
 
 
-# Per-file additions.  qmm_gemm.hip: MFMA accumulators in ordinary VGPRs
-# (with AGPR accumulators the register allocator rotates the loop-carried
-# tiles through copies every iteration of the wide kernel's K loop).
-FILE_FLAGS = {"qmm_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# Per-file additions.  The MFMA kernels: accumulators in ordinary VGPRs (the
+# blockwise kinds scale them with VALU operations, which cannot read AGPRs).
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("qmm_quad.hip", "qmm_quad_half.hip")}
 
 
 def build_vmhip(jobs: int = 8) -> str:

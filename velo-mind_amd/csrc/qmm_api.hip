@@ -8,6 +8,7 @@
 
 #include "a_split.h"
 #include "qmm_kernels.h"
+#include "vm_device.h"
 #include "vm_internal.h"
 
 namespace vmhip {
@@ -54,39 +55,6 @@ __global__ __launch_bounds__(256) void generic_qmm_kernel(const float* __restric
 __global__ void zero_kernel(float* __restrict__ c, int64_t count) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < count) c[i] = 0.0f;
-}
-
-// dtype.h:53-89 (fp16) and :97-107 (bf16), bit for bit.
-__device__ uint16_t f32_to_f16_ref(float f) {
-    const uint32_t x = __float_as_uint(f);
-    const uint32_t sign = (x >> 16) & 0x8000u;
-    const uint32_t raw_e = (x >> 23) & 0xFFu;
-    const uint32_t mant = x & 0x7FFFFFu;
-    if (raw_e == 0xFF) return static_cast<uint16_t>(sign | (mant ? 0x7E00u : 0x7C00u));
-    int e = static_cast<int>(raw_e) - 112;
-    if (e <= 0) {
-        if (e < -10) return static_cast<uint16_t>(sign);
-        uint32_t m = (mant | 0x800000u) >> (1 - e);
-        if ((m & 0x1000u) && (m & 0x2FFFu)) m += 0x2000u;
-        return static_cast<uint16_t>(sign | (m >> 13));
-    }
-    if (e >= 31) return static_cast<uint16_t>(sign | 0x7C00u);
-    uint32_t m = mant;
-    if ((m & 0x1000u) && (m & 0x2FFFu)) {
-        m += 0x2000u;
-        if (m & 0x800000u) {
-            m = 0;
-            if (++e >= 31) return static_cast<uint16_t>(sign | 0x7C00u);
-        }
-    }
-    return static_cast<uint16_t>(sign | (static_cast<uint32_t>(e) << 10) | (m >> 13));
-}
-
-__device__ uint16_t f32_to_bf16_ref(float f) {
-    uint32_t x = __float_as_uint(f);
-    if ((x & 0x7F800000u) == 0x7F800000u && (x & 0x7FFFFFu)) return static_cast<uint16_t>((x >> 16) | 0x40u);
-    x += 0x7FFFu + ((x >> 16) & 1u);
-    return static_cast<uint16_t>(x >> 16);
 }
 
 __global__ void f32_to_half_kernel(const float* __restrict__ src, uint16_t* __restrict__ dst,
@@ -349,7 +317,16 @@ int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale, 
                             static_cast<float*>(c), rows_m, k, n, quant_type, block_size, s);
     if (rows_m == 0 || n == 0) return 0;
 
-    // Stage half operands as fp32: [A | scales | C] in the per-stream buffer.
+    if (k > 0) {
+        const int bs = (quant_type == VM_HIP_QUANT_INT4 && block_size <= 0) ? 32 : block_size;
+        const int rc = gemm_qmm_half(static_cast<const uint16_t*>(a), a_dtype == VM_HIP_DTYPE_BF16,
+                                     reinterpret_cast<const uint8_t*>(wq), scale, scale_dtype != VM_HIP_DTYPE_F32,
+                                     static_cast<uint16_t*>(c), static_cast<int>(rows_m), static_cast<int>(k),
+                                     static_cast<int>(n), quant_type, bs, s);
+        if (rc != VM_HIP_EUNSUPPORTED) return rc;
+    }
+    // Shapes the MFMA kernel does not take: half operands staged as fp32, [A |
+    // scales | C] in the per-stream buffer.
     const int64_t nblk = quant_type == VM_HIP_QUANT_INT4
                              ? (k + (block_size > 0 ? block_size : 32) - 1) / (block_size > 0 ? block_size : 32)
                              : (block_size > 0 ? (k + block_size - 1) / block_size : 1);

@@ -36,16 +36,35 @@ int gemv_qmm_fx_f32(const float* a, const uint8_t* const* wq, const float* const
 int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c, int m, int k,
                  int n, int quant_type, int block_size, hipStream_t stream);
 
-// How the GEMM takes a shape: kind 0 = INT8 per column, 1 = INT8 blockwise,
-// 2 = INT4; `pieces`: A staged in the wide kernel's operand order (else
-// row-major, a_split.h; blockwise scales always take the wide kernel).
-// VM_HIP_EUNSUPPORTED when the GEMM does not take the shape (rows <= 4,
-// K % 32, N % 16, sizes past 32-bit offsets).
+// The same for fp16 or bf16 activations and outputs (any m >= 1); scales fp32
+// or, with scale_half, of the same 16-bit type.
+int gemm_qmm_half(const uint16_t* a, bool bf16, const uint8_t* wq, const void* scale, bool scale_half, uint16_t* c,
+                  int m, int k, int n, int quant_type, int block_size, hipStream_t stream);
+
+// How the GEMM takes A staged by its producer: kind 0 = INT8 per column, 1 =
+// INT8 blockwise, 2 = INT4; `pieces`: operand order (else row-major,
+// a_split.h).  VM_HIP_EUNSUPPORTED for shapes whose producers write fp32
+// (rows <= 4, K % 32, N % 16, sizes past 32-bit offsets); gemm_qmm_f32 and
+// gemm_qmm_half stage ragged K and N themselves.
 struct GemmPlan {
     int kind = 0;
     bool pieces = false;
 };
 int gemm_plan(int m, int k, int n, int quant_type, int block_size, GemmPlan* plan);
+// One call of the MFMA kernel (qmm_quad_impl.h).
+struct GemmOperands {
+    const void* a;
+    int layout;             // 0 operand order, 1 row-major
+    const int* row_exp;     // fp32 only: the rows' staging exponents
+    const uint8_t* wq;
+    const void* scale;
+    bool scale_half;        // scales of A's 16-bit type
+    void* c;
+    int m, k, n, block_size;
+    int kind;               // 0 INT8 per column, 1 INT8 blockwise, 2 INT4
+};
+int quad_qmm_f32(const GemmOperands& o, hipStream_t stream);
+int quad_qmm_half(const GemmOperands& o, bool bf16, hipStream_t stream);
 // The GEMM on A staged by its producer (a_split.h layout for the plan).
 int gemm_qmm_staged_f32(const GemmPlan& plan, const _Float16* ah, const int* row_exp, const uint8_t* wq,
                         const float* scale, float* c, int m, int k, int n, int block_size, hipStream_t stream);

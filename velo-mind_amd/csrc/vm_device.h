@@ -121,4 +121,37 @@ __device__ __forceinline__ unsigned ticket_take(unsigned* counter, unsigned /*co
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float silu_mul_f32(float g, float u) { return (sigmoid_f32(g) * g) * u; }
 
+// dtype.h:53-89 (fp16) and :97-107 (bf16), bit for bit.
+__device__ __forceinline__ uint16_t f32_to_f16_ref(float f) {
+    const uint32_t x = __float_as_uint(f);
+    const uint32_t sign = (x >> 16) & 0x8000u;
+    const uint32_t raw_e = (x >> 23) & 0xFFu;
+    const uint32_t mant = x & 0x7FFFFFu;
+    if (raw_e == 0xFF) return static_cast<uint16_t>(sign | (mant ? 0x7E00u : 0x7C00u));
+    int e = static_cast<int>(raw_e) - 112;
+    if (e <= 0) {
+        if (e < -10) return static_cast<uint16_t>(sign);
+        uint32_t m = (mant | 0x800000u) >> (1 - e);
+        if ((m & 0x1000u) && (m & 0x2FFFu)) m += 0x2000u;
+        return static_cast<uint16_t>(sign | (m >> 13));
+    }
+    if (e >= 31) return static_cast<uint16_t>(sign | 0x7C00u);
+    uint32_t m = mant;
+    if ((m & 0x1000u) && (m & 0x2FFFu)) {
+        m += 0x2000u;
+        if (m & 0x800000u) {
+            m = 0;
+            if (++e >= 31) return static_cast<uint16_t>(sign | 0x7C00u);
+        }
+    }
+    return static_cast<uint16_t>(sign | (static_cast<uint32_t>(e) << 10) | (m >> 13));
+}
+
+__device__ __forceinline__ uint16_t f32_to_bf16_ref(float f) {
+    uint32_t x = __float_as_uint(f);
+    if ((x & 0x7F800000u) == 0x7F800000u && (x & 0x7FFFFFu)) return static_cast<uint16_t>((x >> 16) | 0x40u);
+    x += 0x7FFFu + ((x >> 16) & 1u);
+    return static_cast<uint16_t>(x >> 16);
+}
+
 }  // namespace vmhip
