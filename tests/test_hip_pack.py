@@ -53,6 +53,31 @@ def test_int4_bit_exact(hip, rows, cols, block):
     assert np.array_equal(s.view(np.uint32), s_ref.view(np.uint32))
 
 
+# Whole and partial 32-row groups, blocks that end inside a group of four,
+# 64 x 4-column workgroups with a remainder, and single-column loads (cols % 4).
+@pytest.mark.parametrize("block", [32, 64, 128])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (31, 260), (33, 256), (127, 1028), (129, 257), (300, 67), (2047, 515)])
+def test_int4_row_held_blocks_bit_exact(hip, rows, cols, block):
+    w = _normal(rows, cols, rows * 3 + cols + block)
+    w[:, cols // 2] = 0.0
+    p_ref, s_ref = O.quantize_int4(w, block)
+    p, s = hip.run_pack_int4(w, block)
+    assert np.array_equal(p, p_ref)
+    assert np.array_equal(s.view(np.uint32), s_ref.view(np.uint32))
+
+
+# The two-pass INT8 packer with single-column loads, row groups of 64 with a
+# remainder, and one chunk or the most.
+@pytest.mark.parametrize("rows,cols", [(64, 257), (65, 1001), (2049, 259), (4100, 301)])
+def test_int8_two_pass_odd_columns_bit_exact(hip, rows, cols):
+    w = _normal(rows, cols, rows + cols)
+    w[:, 3] = 0.0
+    q_ref, s_ref = O.quantize_int8(w)
+    q, s = hip.run_pack_int8(w)
+    assert np.array_equal(q, q_ref)
+    assert np.array_equal(s.view(np.uint32), s_ref.view(np.uint32))
+
+
 def test_pack_ties_everywhere(hip):
     # every element lands on an exact .5 after scaling (scale 1/16)
     rng = np.random.default_rng(9)

@@ -52,42 +52,78 @@ __global__ __launch_bounds__(kColsPerWg * kRowGroups) void pack_int8_kernel(
     }
 }
 
-// Two-pass INT8 packing for wide matrices (cols % 4 == 0, aligned): one
-// workgroup of the single-pass kernel scans all rows of 64 columns, a
-// serial chain of loads that leaves the GPU mostly idle (2048 x 5632:
-// 350 us).  Here thread (x, chunk) owns four adjacent columns:
-//   pass 1: the maximum |w| of its columns over one chunk of rows
-//           (16-byte loads, kPackUnroll in flight), one partial per chunk;
-//   pass 2: the column maxima from the partials (max is exact in any
-//           order), then quant.cpp's scale / reciprocal / round / clamp for
-//           its columns over one chunk of rows, four codes per 4-byte store.
-// The comparison `v > m` skips NaN, as the single-pass kernel does.
-constexpr int kPackThreads = 256;
-constexpr int kPackUnroll = 8;
+// V adjacent columns of a row (16-byte loads with V = 4; V = 1 where cols
+// or a pointer rules them out).
+template <int V>
+struct Columns {
+    float e[V];
+};
 
-__global__ __launch_bounds__(kPackThreads) void pack_int8_colmax_kernel(const float* __restrict__ w,
-                                                                        float* __restrict__ part, int64_t rows,
-                                                                        int64_t cols, int64_t rows_per_chunk) {
-    const int64_t c4 = (static_cast<int64_t>(blockIdx.x) * kPackThreads + threadIdx.x) * 4;
-    if (c4 >= cols) return;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * rows_per_chunk;
-    const int64_t r1 = min(rows, r0 + rows_per_chunk);
-    float m[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t r = r0; r < r1; r += kPackUnroll) {
-        float4 v[kPackUnroll];
+// Two-pass INT8 packing (a workgroup of the single-pass kernel scans all rows
+// of 64 columns, a serial chain of loads that leaves the GPU mostly idle).
+// Four waves of 64 V columns:
+//   pass 1: the maximum |w| of the columns over a chunk of rows, kPackRows
+//           loads in flight per wave, the waves' maxima joined in LDS, one
+//           partial per chunk;
+//   pass 2: a wave requests its kPackRows rows, then the column maxima are
+//           joined from the partials (max is exact in any order) while those
+//           are in flight, then quant.cpp's scale / reciprocal / round /
+//           clamp, V codes per store.
+// At most 32 chunks (pass 2 reads every partial).  Against one wave's columns
+// per thread group and no join: 5632 x 2048 55.7 -> 32.1 us, 2048 x 5632 31.1
+// -> 26.2; odd widths, 2048 x 5633, 280 -> 40.
+// The comparison `v > m` skips NaN, as the single-pass kernel does.
+constexpr int kPackRows = 16;
+constexpr int kPackMaxChunks = 32;
+
+template <int V>
+__device__ __forceinline__ void load_rows(const float* __restrict__ w, int64_t r0, int64_t r1, int64_t cols, int64_t c,
+                                          Columns<V> (&x)[kPackRows]) {
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u)
-            v[u] = r + u < r1 ? *reinterpret_cast<const float4*>(w + (r + u) * cols + c4)
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < kPackRows; ++u) {
+        if (r0 + u < r1 && c < cols) {
+            __builtin_memcpy(&x[u], __builtin_assume_aligned(w + (r0 + u) * cols + c, 4 * V), 4 * V);
+        } else {
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u) {
-            const float a[4] = {fabsf(v[u].x), fabsf(v[u].y), fabsf(v[u].z), fabsf(v[u].w)};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (a[e] > m[e]) m[e] = a[e];
+            for (int v = 0; v < V; ++v) x[u].e[v] = 0.0f;
         }
     }
-    *reinterpret_cast<float4*>(part + static_cast<int64_t>(blockIdx.y) * cols + c4) = make_float4(m[0], m[1], m[2], m[3]);
+}
+
+// Column maxima of the four waves, joined in every wave.
+template <int V>
+__device__ __forceinline__ void join_max(float (&m)[V], float (*smax)[64][V], int wave, int lane) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) smax[wave][lane][v] = m[v];
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int v = 0; v < V; ++v) m[v] = smax[g][lane][v] > m[v] ? smax[g][lane][v] : m[v];
+}
+
+template <int V>
+__global__ __launch_bounds__(256) void pack_int8_colmax_kernel(const float* __restrict__ w, float* __restrict__ part,
+                                                               int64_t rows, int64_t cols, int64_t rows_per_chunk) {
+    __shared__ float smax[4][64][V];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * 64 + lane) * V;
+    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * rows_per_chunk;
+    const int64_t r1 = min(rows, r0 + rows_per_chunk);
+    float m[V] = {};
+    for (int64_t r = r0 + wave * kPackRows; r < r1; r += 4 * kPackRows) {
+        Columns<V> x[kPackRows];
+        load_rows<V>(w, r, r1, cols, c, x);
+#pragma unroll
+        for (int u = 0; u < kPackRows; ++u)
+#pragma unroll
+            for (int v = 0; v < V; ++v) m[v] = fabsf(x[u].e[v]) > m[v] ? fabsf(x[u].e[v]) : m[v];
+    }
+    join_max<V>(m, smax, wave, lane);
+    if (wave == 0 && c < cols) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) part[static_cast<int64_t>(blockIdx.y) * cols + c + v] = m[v];
+    }
 }
 
 __device__ __forceinline__ uint32_t int8_code(float x, float inv) {
@@ -96,49 +132,43 @@ __device__ __forceinline__ uint32_t int8_code(float x, float inv) {
     return static_cast<uint32_t>(static_cast<uint8_t>(static_cast<int8_t>(v)));
 }
 
-__global__ __launch_bounds__(kPackThreads) void pack_int8_quantize_kernel(
-    const float* __restrict__ w, const float* __restrict__ part, int chunks, int8_t* __restrict__ q,
-    float* __restrict__ scale, int64_t rows, int64_t cols, int64_t rows_per_chunk) {
-    const int64_t c4 = (static_cast<int64_t>(blockIdx.x) * kPackThreads + threadIdx.x) * 4;
-    if (c4 >= cols) return;
-    float amax[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int i0 = 0; i0 < chunks; i0 += kPackUnroll) {
-        float4 pv[kPackUnroll];
+template <int V>
+__global__ __launch_bounds__(256) void pack_int8_quantize_kernel(const float* __restrict__ w,
+                                                                 const float* __restrict__ part, int chunks,
+                                                                 int8_t* __restrict__ q, float* __restrict__ scale,
+                                                                 int64_t rows, int64_t cols) {
+    __shared__ float smax[4][64][V];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * 64 + lane) * V;
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.y) * 4 + wave) * kPackRows;
+    Columns<V> x[kPackRows];
+    load_rows<V>(w, r0, rows, cols, c, x);
+    float m[V] = {};
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u)
-            pv[u] = i0 + u < chunks ? *reinterpret_cast<const float4*>(part + static_cast<int64_t>(i0 + u) * cols + c4)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < kPackMaxChunks / 4; ++i) {
+        const int ch = wave + 4 * i;
+        if (ch < chunks && c < cols) {
+            Columns<V> p;
+            __builtin_memcpy(&p, part + static_cast<int64_t>(ch) * cols + c, 4 * V);
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u) {
-            const float a[4] = {pv[u].x, pv[u].y, pv[u].z, pv[u].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (a[e] > amax[e]) amax[e] = a[e];
+            for (int v = 0; v < V; ++v) m[v] = p.e[v] > m[v] ? p.e[v] : m[v];
         }
     }
-    float inv[4];
-    float sc[4];
+    join_max<V>(m, smax, wave, lane);
+    if (c >= cols) return;
+    float inv[V];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        sc[e] = amax[e] > 0.0f ? amax[e] / 127.0f : 1.0f;   // quant.cpp:94-96
-        inv[e] = 1.0f / sc[e];
+    for (int v = 0; v < V; ++v) {
+        const float sc = m[v] > 0.0f ? m[v] / 127.0f : 1.0f;   // quant.cpp:94-96
+        inv[v] = 1.0f / sc;
+        if (blockIdx.y == 0 && wave == 0) scale[c + v] = sc;
     }
-    if (blockIdx.y == 0) *reinterpret_cast<float4*>(scale + c4) = make_float4(sc[0], sc[1], sc[2], sc[3]);
-    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * rows_per_chunk;
-    const int64_t r1 = min(rows, r0 + rows_per_chunk);
-    for (int64_t r = r0; r < r1; r += kPackUnroll) {
-        float4 v[kPackUnroll];
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u)
-            v[u] = r + u < r1 ? *reinterpret_cast<const float4*>(w + (r + u) * cols + c4)
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < kPackRows; ++u) {
+        uint32_t b = 0;
 #pragma unroll
-        for (int u = 0; u < kPackUnroll; ++u) {
-            if (r + u >= r1) break;
-            const uint32_t word = int8_code(v[u].x, inv[0]) | (int8_code(v[u].y, inv[1]) << 8) |
-                                  (int8_code(v[u].z, inv[2]) << 16) | (int8_code(v[u].w, inv[3]) << 24);
-            *reinterpret_cast<uint32_t*>(q + (r + u) * cols + c4) = word;
-        }
+        for (int v = 0; v < V; ++v) b |= int8_code(x[u].e[v], inv[v]) << (8 * v);
+        if (r0 + u < rows) __builtin_memcpy(__builtin_assume_aligned(q + (r0 + u) * cols + c, V), &b, V);
     }
 }
 
@@ -148,7 +178,76 @@ __device__ __forceinline__ unsigned int4_code(float x, float inv) {
     return static_cast<unsigned>(static_cast<int8_t>(v)) & 0xFu;
 }
 
-// One thread per (scale block, column); blocks are even, so every packed
+// INT4 blocks of 32 * G rows, G a power of two up to 4: bandwidth-bound, so
+// the matrix is read once.  A thread holds 32 rows of V adjacent columns
+// (all its loads in flight at once, 16 bytes each with V = 4), finds their
+// maxima, the G waves of a block exchange theirs through LDS, and the held
+// values are quantized and stored V packed bytes at a time.  Four waves
+// cover 4 / G blocks.  2048 x 32000, blocks of 32: 67 us (4.4 TB/s; a
+// copy reaches 5.1), against 113 with a thread per block and column, which
+// reads 4 bytes a lane, twice.
+template <int V, int G>
+__global__ __launch_bounds__(256) void pack_int4_rows_kernel(const float* __restrict__ w, uint8_t* __restrict__ packed,
+                                                             float* __restrict__ scale, int64_t rows, int64_t cols) {
+    constexpr int R = 32;
+    __shared__ float smax[4][64][V];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * 64 + lane) * V;
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.y) * 4 + wave) * R;
+    const bool in = c < cols;
+    Columns<V> x[R];
+    const float* src = w + r0 * cols + c;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (in && r0 + r < rows) {
+            __builtin_memcpy(&x[r], __builtin_assume_aligned(src + r * cols, 4 * V), 4 * V);
+        } else {
+#pragma unroll
+            for (int v = 0; v < V; ++v) x[r].e[v] = 0.0f;
+        }
+    }
+    float amax[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) amax[v] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < V; ++v) amax[v] = fabsf(x[r].e[v]) > amax[v] ? fabsf(x[r].e[v]) : amax[v];   // skips NaN
+    if constexpr (G > 1) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) smax[wave][lane][v] = amax[v];
+        __syncthreads();
+        const int first = wave & ~(G - 1);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            float m = smax[first][lane][v];
+#pragma unroll
+            for (int g = 1; g < G; ++g) m = smax[first + g][lane][v] > m ? smax[first + g][lane][v] : m;
+            amax[v] = m;
+        }
+    }
+    if (!in || r0 >= rows) return;
+    Columns<V> s;
+    float inv[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        s.e[v] = amax[v] > 0.0f ? amax[v] / 7.0f : 1.0f;
+        inv[v] = 1.0f / s.e[v];
+    }
+    if (wave % G == 0)
+        __builtin_memcpy(__builtin_assume_aligned(scale + r0 / (R * G) * cols + c, 4 * V), &s, 4 * V);
+    uint8_t* dst = packed + r0 / 2 * cols + c;
+#pragma unroll
+    for (int r = 0; r < R; r += 2) {
+        uint32_t b = 0;
+#pragma unroll
+        for (int v = 0; v < V; ++v)   // rows past the matrix hold zeros, code 0
+            b |= (int4_code(x[r].e[v], inv[v]) | int4_code(x[r + 1].e[v], inv[v]) << 4) << (8 * v);
+        if (r0 + r < rows) __builtin_memcpy(__builtin_assume_aligned(dst + r / 2 * cols, V), &b, V);
+    }
+}
+
+// Any other block size: one thread per (scale block, column); blocks are even, so every packed
 // byte belongs to exactly one thread.
 __global__ __launch_bounds__(256) void pack_int4_kernel(const float* __restrict__ w,
                                                         uint8_t* __restrict__ packed,
@@ -252,26 +351,33 @@ int vm_hip_pack_int8(const float* w, int8_t* q, float* scale, int64_t rows, int6
     if (!w || !q || !scale) return fail_inval("vm_hip_pack_int8: null pointer");
     VM_TRY(injected_failure("QuantizePack", "launch"));
     auto s = static_cast<hipStream_t>(stream);
-    // Two passes for matrices wide and tall enough to fill the GPU, when
-    // 16-byte loads apply and the stream is not being captured (the row
-    // partials use the stream's workspace, sized here).
+    // Two passes for matrices wide and tall enough to fill the GPU, when the
+    // stream is not being captured (the row partials use the stream's
+    // workspace, sized here) and the second pass's grid holds the rows.
     const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
-                     reinterpret_cast<uintptr_t>(q) % 4 == 0 && reinterpret_cast<uintptr_t>(scale) % 16 == 0;
+                     reinterpret_cast<uintptr_t>(q) % 4 == 0;
+    const int64_t row_groups = (rows + 4 * kPackRows - 1) / (4 * kPackRows);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (s) (void)hipStreamIsCapturing(s, &cap);
-    if (vec && rows >= 64 && cols >= 256 && cap == hipStreamCaptureStatusNone) {
-        const int64_t col_groups = (cols / 4 + kPackThreads - 1) / kPackThreads;
-        // about 512 workgroups per pass, at least 32 rows and at most 64 chunks
-        int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((512 + col_groups - 1) / col_groups, rows / 32));
-        chunks = std::min<int64_t>(chunks, 64);   // pass 2 reads every chunk's partial
-        const int64_t rpc = (rows + chunks - 1) / chunks;
+    if (rows >= 64 && cols >= 256 && row_groups <= 65535 && cap == hipStreamCaptureStatusNone) {
+        const int64_t col_groups = (cols + (vec ? 255 : 63)) / (vec ? 256 : 64);
+        // about 1024 workgroups, whole steps of 64 rows each
+        int64_t chunks = std::min<int64_t>({(1024 + col_groups - 1) / col_groups, row_groups, kPackMaxChunks});
+        const int64_t rpc = (row_groups + chunks - 1) / chunks * (4 * kPackRows);
         chunks = (rows + rpc - 1) / rpc;
         Workspace ws{};
         VM_TRY(get_workspace(s, static_cast<std::size_t>(chunks * cols), 0, &ws));
         const dim3 grid(static_cast<unsigned>(col_groups), static_cast<unsigned>(chunks));
-        hipLaunchKernelGGL(pack_int8_colmax_kernel, grid, dim3(kPackThreads), 0, s, w, ws.partials, rows, cols, rpc);
-        hipLaunchKernelGGL(pack_int8_quantize_kernel, grid, dim3(kPackThreads), 0, s, w, ws.partials,
-                           static_cast<int>(chunks), q, scale, rows, cols, rpc);
+        const dim3 grid2(static_cast<unsigned>(col_groups), static_cast<unsigned>(row_groups));
+        if (vec) {
+            hipLaunchKernelGGL(pack_int8_colmax_kernel<4>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
+            hipLaunchKernelGGL(pack_int8_quantize_kernel<4>, grid2, dim3(256), 0, s, w, ws.partials,
+                               static_cast<int>(chunks), q, scale, rows, cols);
+        } else {
+            hipLaunchKernelGGL(pack_int8_colmax_kernel<1>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
+            hipLaunchKernelGGL(pack_int8_quantize_kernel<1>, grid2, dim3(256), 0, s, w, ws.partials,
+                               static_cast<int>(chunks), q, scale, rows, cols);
+        }
         return check_launch("QuantizePack", s);
     }
     hipLaunchKernelGGL(pack_int8_kernel, dim3(grid_1d(cols, kColsPerWg)), dim3(kColsPerWg * kRowGroups),
@@ -289,6 +395,25 @@ int vm_hip_pack_int4(const float* w, uint8_t* packed, float* scale, int64_t rows
     const int64_t nblk = (rows + block - 1) / block;
     if (nblk > 65535) return fail_inval("vm_hip_pack_int4: too many scale blocks");
     auto s = static_cast<hipStream_t>(stream);
+    if (block == 32 || block == 64 || block == 128) {
+        const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                         reinterpret_cast<uintptr_t>(packed) % 4 == 0 && reinterpret_cast<uintptr_t>(scale) % 16 == 0;
+        const int64_t groups = (rows + 127) / 128;   // (at most 65535, as the blocks above)
+#define VM_PACK4(VX, GX)                                                                                             \
+    hipLaunchKernelGGL((pack_int4_rows_kernel<VX, GX>), dim3(grid_1d(cols, 64 * VX), static_cast<unsigned>(groups)), \
+                       dim3(256), 0, s, w, packed, scale, rows, cols)
+        if (vec) {
+            if (block == 32) VM_PACK4(4, 1);
+            else if (block == 64) VM_PACK4(4, 2);
+            else VM_PACK4(4, 4);
+        } else {
+            if (block == 32) VM_PACK4(1, 1);
+            else if (block == 64) VM_PACK4(1, 2);
+            else VM_PACK4(1, 4);
+        }
+#undef VM_PACK4
+        return check_launch("QuantizePack", s);
+    }
     hipLaunchKernelGGL(pack_int4_kernel, dim3(grid_1d(cols, 256), static_cast<unsigned>(nblk)), dim3(256),
                        0, s, w, packed, scale, rows, cols, block);
     return check_launch("QuantizePack", s);
