@@ -54,6 +54,27 @@ def test_ragged_fp32(hip, kind, block, m, k, n):
     assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * mag + 1e-30)
 
 
+@pytest.mark.parametrize("kind,block", [("int8", 0), ("int8", 24), ("int4", 32), ("int4", 8)])
+@pytest.mark.parametrize("m", [1, 3])
+@pytest.mark.parametrize("k,n", [(31, 17), (64, 31), (576, 257), (2048, 515), (2048, 5633), (300, 26000 + 7), (5632, 2049)])
+def test_ragged_gemv(hip, kind, block, m, k, n):
+    # up to four rows: the 16-column groups of every tile width and split of
+    # the decode kernel, the last one moved back inside the row
+    rng = np.random.default_rng(m + k + n + block)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    print(f"case ragged gemv {kind} block={block} m={m} k={k} n={n}", flush=True)
+    wd = _dense(v, s, block)
+    bound = 2 * k * 2.0 ** -24 * 1.01 * (np.abs(x.astype(np.float64)) @ np.abs(wd)) + 1e-30
+    for shift in (0, 1):   # codes at an odd address too
+        buf = np.zeros(q.nbytes + 1, np.int8)
+        buf[shift:shift + q.nbytes] = q.view(np.int8).reshape(-1)
+        da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (x, buf, s, np.zeros((m, n), np.float32)))
+        hip.qmm_f32(da.addr, dq.addr + shift, ds.addr, dc.addr, m, k, n, qt, block)
+        out = dc.download(np.float32, (m, n)).astype(np.float64)
+        assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= bound)
+
+
 def _bits(x, bf16):
     return O.f32_to_bf16_bits(x) if bf16 else O.f32_to_f16_bits(x)
 

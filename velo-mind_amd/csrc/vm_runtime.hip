@@ -180,8 +180,6 @@ int get_workspace(hipStream_t stream, std::size_t partial_floats, std::size_t co
     return 0;
 }
 
-bool scratch_holds(std::size_t bytes) { return !t_fixed || bytes + 256 <= t_fixed->partial_floats * sizeof(float); }
-
 int get_aux(hipStream_t stream, std::size_t bytes, void** out) {
     bytes = (bytes + 255) & ~std::size_t(255);
     if (FixedRegion* f = t_fixed) {
