@@ -21,9 +21,11 @@
 //       order, times codes that are exact in the same type.
 // Work
 //   wave       BM = TILE * MT rows x NT = 4 * TILE columns over its own run of
-//              32-row K chunks; the waves of a workgroup split K, so the main
-//              loop has no barrier and no LDS traffic
-//   workgroup  W waves on one tile; their sums meet in LDS in wave order
+//              32-row K chunks; waves split K, so the main loop has no barrier
+//              and no LDS traffic
+//   workgroup  W waves: NW side by side in N (large calls: A's lines are then
+//              shared in L1), KW splitting K; the KW sums meet in LDS in wave
+//              order
 //   split      further K splits across workgroups; partial tiles go to the
 //              stream's workspace and the last workgroup of a tile adds them
 //              in split order (results do not depend on scheduling)
@@ -199,12 +201,14 @@ struct QuadArgs {
 };
 
 // KIND: 0 = INT8 per column, 1 = INT8 blockwise, 2 = INT4 blockwise.
-template <int KIND, int TILE, int MT, int W, int AM, int EL, bool SH, int D>
+template <int KIND, int TILE, int MT, int W, int NW, int AM, int EL, bool SH, int D>
 struct QuadCfg {
     using M = Mfma<TILE>;
     static constexpr int PARTS = EL == EL_F32 ? 2 : 1;
     static constexpr int BM = TILE * MT;
-    static constexpr int NT = 4 * TILE;
+    static constexpr int KW = W / NW;                     // waves that split K
+    static constexpr int WT = 4 * TILE;                   // columns of a wave
+    static constexpr int NT = NW * WT;                    // and of the workgroup
     // K rows per pipeline stage: a scale block's granularity, else one MFMA
     static constexpr int kChunk = KIND != 0 ? 32 : M::kK;
     static constexpr int Q = kChunk / M::kK;              // MFMA K steps per chunk
@@ -217,14 +221,14 @@ struct QuadCfg {
     static constexpr int kRegs = kItems * 4 + D * (MT * Q * 4 * PARTS + Q * kWords + (kBlock ? 4 : 0)) +
                                  (kBlock ? 2 * MT * M::kElems : 0) + Q * 8 + 16;
     static constexpr int kWavesPerEu = W >= 8 ? 2 : kRegs <= 256 ? 2 : 1;
-    static_assert(kItems % kPhase == 0 && (kPhase % W == 0 || kPhase < W), "phases split the items, waves split a phase");
+    static_assert(kItems % kPhase == 0 && (kPhase % KW == 0 || kPhase < KW), "phases split the items, waves split a phase");
 };
 
-template <int KIND, int TILE, int MT, int W, int AM, int EL, bool SH, int D>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(QuadCfg<KIND, TILE, MT, W, AM, EL, SH, D>::kWavesPerEu,
-                                                                        QuadCfg<KIND, TILE, MT, W, AM, EL, SH, D>::kWavesPerEu)))
+template <int KIND, int TILE, int MT, int W, int NW, int AM, int EL, bool SH, int D>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(QuadCfg<KIND, TILE, MT, W, NW, AM, EL, SH, D>::kWavesPerEu,
+                                                                        QuadCfg<KIND, TILE, MT, W, NW, AM, EL, SH, D>::kWavesPerEu)))
 void qmm_quad_kernel(const QuadArgs g) {
-    using C = QuadCfg<KIND, TILE, MT, W, AM, EL, SH, D>;
+    using C = QuadCfg<KIND, TILE, MT, W, NW, AM, EL, SH, D>;
     using M = typename C::M;
     using Acc = typename M::Acc;
     constexpr int PARTS = C::PARTS;
@@ -252,9 +256,10 @@ void qmm_quad_kernel(const QuadArgs g) {
     const int m0 = tile_y * C::BM;
     // The lane's four columns; a quad that would cross the row's end moves
     // back to end with it (its first columns are then the quad before's).
-    const int col = tile_x * C::NT + 4 * lc;
+    const int wn = wave % NW, wk = wave / NW;
+    const int col = tile_x * C::NT + wn * C::WT + 4 * lc;
     const int cs = min(col, n - 4);
-    const int c_begin = min((split * W + wave) * g.chunks_per_wave, g.chunks);
+    const int c_begin = min((split * C::KW + wk) * g.chunks_per_wave, g.chunks);
     const int c_end = min(c_begin + g.chunks_per_wave, g.chunks);
 
     const __amdgpu_buffer_rsrc_t ars = buffer_rsrc(g.a, g.a_bytes);
@@ -522,8 +527,8 @@ void qmm_quad_kernel(const QuadArgs g) {
     // partial tiles: [tile][split][item][lane] float4
     const int tile = tile_x * g.tiles_m + tile_y;
     const __amdgpu_buffer_rsrc_t prs =
-        buffer_rsrc(g.partials + static_cast<int64_t>(tile) * splits * (C::kItems * 256), 0x7fffffff);
-    constexpr int kOwn = (C::kPhase + W - 1) / W;   // items of a phase that a wave adds up
+        buffer_rsrc(g.partials + static_cast<int64_t>(tile * NW + wn) * splits * (C::kItems * 256), 0x7fffffff);
+    constexpr int kOwn = (C::kPhase + C::KW - 1) / C::KW;   // items of a phase that a wave adds up
     for (int ph = 0; ph < C::kItems; ph += C::kPhase) {
         if (ph) __syncthreads();
 #pragma unroll
@@ -536,12 +541,12 @@ void qmm_quad_kernel(const QuadArgs g) {
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kOwn; ++j) {
-            const int i = wave * kOwn + j;
-            if (C::kPhase < W && i >= C::kPhase) break;
-            float4 v = red[i * 64 + lane];
+            const int i = wk * kOwn + j;
+            if (C::kPhase < C::KW && i >= C::kPhase) break;
+            float4 v = red[(wn * C::kPhase + i) * 64 + lane];
 #pragma unroll
-            for (int w = 1; w < W; ++w) {
-                const float4 x = red[(w * C::kPhase + i) * 64 + lane];
+            for (int w = 1; w < C::KW; ++w) {
+                const float4 x = red[((w * NW + wn) * C::kPhase + i) * 64 + lane];
                 v.x += x.x;
                 v.y += x.y;
                 v.z += x.z;
@@ -571,7 +576,7 @@ void qmm_quad_kernel(const QuadArgs g) {
     if (tid == 0) ticket = ticket_take(&g.counters[tile], static_cast<unsigned>(splits));
     __syncthreads();
     if (ticket != static_cast<unsigned>(splits - 1)) return;
-    for (int item = wave; item < C::kItems; item += W) {
+    for (int item = wk; item < C::kItems; item += C::KW) {
         const int row = m0 + (item / M::kElems) * TILE + M::row(item % M::kElems, lg);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int s0 = 0; s0 < splits; s0 += 4) {
@@ -594,9 +599,9 @@ void qmm_quad_kernel(const QuadArgs g) {
     if (tid == 0) __hip_atomic_store(&g.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int KIND, int TILE, int MT, int W, int AM, int EL, bool SH, int D>
+template <int KIND, int TILE, int MT, int W, int NW, int AM, int EL, bool SH, int D>
 int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
-    using C = QuadCfg<KIND, TILE, MT, W, AM, EL, SH, D>;
+    using C = QuadCfg<KIND, TILE, MT, W, NW, AM, EL, SH, D>;
     QuadArgs g{};
     g.a = o.a;
     g.row_exp = o.row_exp;
@@ -611,12 +616,12 @@ int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
     g.block_chunks = KIND == 0 ? 1 : o.block_size / C::kChunk;
     g.tiles_n = (o.n + C::NT - 1) / C::NT;
     g.tiles_m = (o.m + C::BM - 1) / C::BM;
-    const int units = splits * W;
+    const int units = splits * C::KW;
     g.chunks_per_wave = (g.chunks + units - 1) / units;
-    splits = (g.chunks + g.chunks_per_wave * W - 1) / (g.chunks_per_wave * W);
+    splits = (g.chunks + g.chunks_per_wave * C::KW - 1) / (g.chunks_per_wave * C::KW);
     Workspace ws{};
     const std::size_t tiles = static_cast<std::size_t>(g.tiles_n) * g.tiles_m;
-    if (splits > 1) VM_TRY(get_workspace(stream, tiles * splits * (C::kItems * 256), tiles, &ws));
+    if (splits > 1) VM_TRY(get_workspace(stream, tiles * NW * splits * (C::kItems * 256), tiles, &ws));
     g.partials = ws.partials;
     g.counters = ws.counters;
     const int64_t rows = AM == AM_PIECES ? (static_cast<int64_t>(o.m) + 31) / 32 * 32 : o.m;
@@ -626,7 +631,7 @@ int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
     g.code_bytes = static_cast<uint32_t>((KIND == 2 ? (static_cast<int64_t>(o.k) + 1) / 2 : static_cast<int64_t>(o.k)) * o.n);
     g.scale_bytes = static_cast<uint32_t>(nblk * o.n * (SH ? 2 : 4));
     g.c_vec = o.n % 4 == 0 && reinterpret_cast<uintptr_t>(o.c) % 8 == 0 ? 1 : 0;
-    hipLaunchKernelGGL((qmm_quad_kernel<KIND, TILE, MT, W, AM, EL, SH, D>), dim3(static_cast<unsigned>(tiles * splits)),
+    hipLaunchKernelGGL((qmm_quad_kernel<KIND, TILE, MT, W, NW, AM, EL, SH, D>), dim3(static_cast<unsigned>(tiles * splits)),
                        dim3(64 * W), 0, stream, g);
     return check_launch("QuantizedMatMul", stream);
 }
@@ -634,6 +639,7 @@ int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
 // Tile, waves and K splits of a call.
 struct QuadConfig {
     int tile, mt, waves, splits;
+    bool pair = false;   // two waves side by side in N, two in K
 };
 
 // Chosen from sweeps of every tile, wave count and 1 - 12 splits on MI355X
@@ -650,6 +656,11 @@ struct QuadConfig {
 //     column feeds two row tiles (M = 512, 2048 x 11264 50.8 us against 59.7;
 //     blockwise kinds lack the registers: M = 512, 2048 x 5632 INT4 46 us
 //     against 36).
+//   * two waves side by side in N, sharing A's lines in L1, where the tiles are
+//     many enough to do with two waves in K: blockwise above 512 rows from 600 tiles
+//     of 32 x 256 (M = 1024, 2048 x 5632 INT4 76.5 -> 65.8 us; M = 512, 2048 x
+//     11264 64.1 -> 61 to 66, 2048 x 5632 41 -> 43.5), 64-row tiles from 1200 (M = 1024, 2048 x 11264
+//     INT8 102 -> 95; 704 tiles 51.7 -> 55.7).
 //   * eight waves per tile; four once the tiles alone fill the GPU (more than
 //     260), or when a 16-row tile's K is too short for eight (576 x 1536).
 //   * K splits only where the tiles leave compute units idle: 16-row tiles
@@ -660,7 +671,8 @@ struct QuadConfig {
 // A call's fp32 partial tiles and staged A stay below 14 MiB, the room that
 // the no-allocation entry point has, so that both choose alike.
 // VELOMIND_GEMM_WIDE="BM,BN,S,D[,G]" or VELOMIND_GEMM_CFG="BM,BN,S[,D]" force
-// the row tile (nearest to BM), S splits and, with D or G of 2, eight waves.
+// the row tile (nearest to BM), paired waves with BN of 256 or more, S splits
+// and, with D or G of 2, eight waves.
 template <int KIND, int AM, int EL>
 QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
     const double code_bytes = (KIND == 2 ? 0.5 : 1.0) * k * n;
@@ -680,6 +692,10 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
         if (KIND == 0 && AM == AM_PIECES && tiles64 >= 170 && (m + 63) / 64 * 64 <= (m + 31) / 32 * 36) {
             c.mt = 2;
             c.waves = 4;
+            c.pair = tiles64 >= 1200;
+        } else if (KIND != 0 && AM == AM_PIECES && m > 512 && tiles_of(32, 256) >= 600) {
+            c.waves = 4;
+            c.pair = true;
         } else {
             const long tiles = tiles_of(32, 128);
             if (tiles > 260) c.waves = 4;
@@ -697,6 +713,7 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
     if (got >= 3 && bm >= 16 && s >= 1 && s <= 16) {
         c.tile = bm <= 16 ? 16 : 32;
         c.mt = bm >= 128 && KIND == 0 && AM == AM_PIECES ? 2 : 1;
+        c.pair = bn >= 256 && AM == AM_PIECES && c.tile == 32 && (c.mt == 2 || KIND != 0);
         c.waves = c.mt == 1 && (d == 2 || g == 2) ? 8 : 4;
         c.splits = s;
     }
@@ -708,13 +725,19 @@ int launch_mode(const GemmOperands& o, hipStream_t s) {
     const std::size_t a_bytes = AM == AM_PIECES ? a_stage_bytes(o.m, (o.k + 31) / 32 * 32, true) : 0;
     const QuadConfig c = choose_quad<KIND, AM, EL>(o.m, o.k, o.n, a_bytes);
     if (c.tile == 16) {
-        if (c.waves == 4) return launch_quad<KIND, 16, 1, 4, AM, EL, SH, 3>(o, c.splits, s);
-        return launch_quad<KIND, 16, 1, 8, AM, EL, SH, 3>(o, c.splits, s);
+        if (c.waves == 4) return launch_quad<KIND, 16, 1, 4, 1, AM, EL, SH, 3>(o, c.splits, s);
+        return launch_quad<KIND, 16, 1, 8, 1, AM, EL, SH, 3>(o, c.splits, s);
     }
-    if constexpr (KIND == 0 && AM == AM_PIECES)
-        if (c.mt == 2) return launch_quad<KIND, 32, 2, 4, AM, EL, SH, 4>(o, c.splits, s);
-    if (c.waves == 4) return launch_quad<KIND, 32, 1, 4, AM, EL, SH, 3>(o, c.splits, s);
-    return launch_quad<KIND, 32, 1, 8, AM, EL, SH, 3>(o, c.splits, s);
+    if constexpr (AM == AM_PIECES) {
+        if constexpr (KIND == 0)
+            if (c.mt == 2)
+                return c.pair ? launch_quad<KIND, 32, 2, 4, 2, AM, EL, SH, 4>(o, c.splits, s)
+                              : launch_quad<KIND, 32, 2, 4, 1, AM, EL, SH, 4>(o, c.splits, s);
+        if constexpr (KIND != 0)
+            if (c.pair) return launch_quad<KIND, 32, 1, 4, 2, AM, EL, SH, 3>(o, c.splits, s);
+    }
+    if (c.waves == 4) return launch_quad<KIND, 32, 1, 4, 1, AM, EL, SH, 3>(o, c.splits, s);
+    return launch_quad<KIND, 32, 1, 8, 1, AM, EL, SH, 3>(o, c.splits, s);
 }
 
 template <int AM, int EL, bool SH>
