@@ -3,31 +3,35 @@
 // rows.
 //
 // A workgroup of four waves takes QR = 16 RW query rows of one head: wave w
-// owns rows 16 (w % RW) .. +15 and key group w / RW of KS.  The keys go by
-// in steps of KS 64-key tiles staged in LDS; group g runs its online
-// softmax over tile g of each step, and the groups' (max, sum, output)
-// triples are merged through LDS at the end.  Splitting the keys cuts the
-// longest chain of dependent MFMAs (the last query rows see every key) by
-// KS; the grid is one-dimensional with the query tiles that see the most
-// keys first, so the workgroups dispatched last are the short ones.
+// owns rows 16 (w % RW) .. +15 and, of the KS key groups, group w / RW: the
+// blocks of KB keys whose number is w / RW modulo KS.  A wave reads its K and
+// V blocks from global memory straight into MFMA operand registers, one
+// block ahead, so the loop has no LDS traffic and no barrier, and two waves
+// per SIMD hide each other's softmax; the groups' (max, sum, output) triples
+// are merged through LDS at the end.  (Staging K and V in LDS for the whole
+// workgroup took 20 us at 512 x 512, 15 heads of 64, most of it waiting at
+// its two barriers per step; three-way bf16 splits of every operand on the
+// 16-bit matrix cores there, 24 us: the splitting costs what it saves.)
+// The grid is one-dimensional with the query tiles that see the most keys
+// first, so the workgroups dispatched last are the short ones.
 //
 // v_mfma_f32_16x16x4_f32 (fp32 inputs and accumulation, so no precision is
 // given up against the fp32 reference) holds A[i][k] in lane i + 16k,
 // B[k][j] in lane j + 16k and D[i][j] in lane j + 16 (i / 4), element i % 4.
-// Scores are computed transposed, S^T = K Q^T, so lane (row r = lane % 16,
-// group g = lane / 16) holds row r's scores for keys 16b + 4g + e: exactly
-// the A operand of P V once the product's reduction index is ordered as
-// key(s, k) = 16 (s / 4) + 4k + s % 4 (the order of a sum's terms is free).
-// Output column j of MFMA tile db is dim 64 (db / 4) + 4 j + db % 4, so that
-// a lane's four V operands of a key are one 16-byte LDS read, and its
-// results one 16-byte store.  Four independent accumulators alternate in
-// both products.  Row statistics live in the lanes of row r (shared across
-// the four groups); output row 4g + e fetches its factor from lane 4g + e.
+// Scores are computed transposed, S^T = K Q^T, four dims 16 c + 4 k + e at a
+// time (lane group k holds four adjacent dims: one 16-byte load); lane (row r
+// = lane % 16, group g = lane / 16) then holds row r's scores for keys 16b +
+// 4g + e: exactly the A operand of P V once the product's reduction index is
+// ordered as key(s, k) = 16 (s / 4) + 4k + s % 4 (the order of a sum's terms
+// is free).  Output column j of MFMA tile db is dim 64 (db / 4) + 4 j + db %
+// 4, so that a lane's four V operands of a key are one 16-byte load, and its
+// results one 16-byte store.  Row statistics live in the lanes of row r
+// (shared across the four groups); output row 4g + e fetches its factor from
+// lane 4g + e.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
-#include <cstdlib>
 
 #include "attention.h"
 #include "vm_internal.h"
@@ -38,7 +42,6 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kTile = 64;   // keys per tile (one key group's share of a step)
 
 // e^x for x <= 0: 2^h with h = x log2 e rounded, times e^l for what the
 // rounding and log2 e's own lost (the error of 2^h alone grows with |x|).
@@ -52,24 +55,29 @@ __device__ __forceinline__ float exp_nonpos(float x) {
 }
 
 template <int D, int RW, int KS>
-__global__ __launch_bounds__(kThreads) void attention_mfma_kernel(const AttentionCall a) {
-    static_assert(D == 64 || D == 128, "64-dim slabs, 16 dims per lane group");
-    static_assert(RW * KS == 4, "four waves");
+__global__ __launch_bounds__(kThreads, 2) void attention_mfma_kernel(const AttentionCall a, int fold) {
+    static_assert(D == 64 || D == 128, "64-dim slabs");
+    static_assert(RW * KS == 4 && KS > 1, "four waves");
     constexpr int H = D / 64;          // 64-dim slabs
-    constexpr int ST = kTile * KS;     // keys per step
-    constexpr int PITCH = D + 4;       // LDS row pitch in floats (conflict-free 16-byte reads)
+    constexpr int KB = 32 / H;         // keys per block: K and V of two blocks fit the registers
+    constexpr int NB = KB / 16;        // 16-key MFMA tiles of a block
+    constexpr int NC = D / 16;         // 16-dim groups
+    constexpr int NS = KB / 4;         // reduction steps of P V
     constexpr int QR = 16 * RW;        // query rows per workgroup
-    extern __shared__ __align__(16) float smem[];
-    float* sk = smem;                  // [ST][PITCH]
-    float* sv = smem + ST * PITCH;
-    __shared__ int v_special[2];       // whether the step's V holds an infinity or NaN, by step parity
     const int tiles = (a.rows + QR - 1) / QR;
     const int bh_count = a.batch * a.heads;
-    const int bh = static_cast<int>(blockIdx.x) % bh_count;
+    // Tiles in descending order of the keys they see; of a grid that fits the
+    // GPU two workgroups to a compute unit, the second one per unit comes in
+    // ascending order, so that a unit's two together see about as many as any
+    // other's (512 cached rows, 32 heads: 26.2 -> 22.7 us).
+    int order = static_cast<int>(blockIdx.x);
+    if (fold > 0 && order >= fold) order = fold + static_cast<int>(gridDim.x) - 1 - order;
+    const int bh = order % bh_count;
     const int bkv = bh / a.heads * a.kv_heads + bh % a.heads / (a.heads / a.kv_heads);
-    const int r0 = (tiles - 1 - static_cast<int>(blockIdx.x) / bh_count) * QR;
+    const int r0 = (tiles - 1 - order / bh_count) * QR;
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave % RW, kg = wave / RW;   // row block, key group
     const int lr = lane & 15, lg = lane >> 4;
     const int p0 = a.pos ? a.pos[0] : a.keys - a.rows;   // position of query row 0
@@ -84,103 +92,66 @@ __global__ __launch_bounds__(kThreads) void attention_mfma_kernel(const Attentio
     const int wave_last = r0 + 16 * wr >= a.rows ? -1 : a.causal ? min(p0 + row_end, n_keys - 1) : n_keys - 1;
     const int wave_first = a.causal ? min(p0 + r0 + 16 * wr, n_keys - 1) : n_keys - 1;
 
-    // Q fragment: Q[qrow][64 h + 16 lg + s], s = 0..15.
-    float4 qf[H][4];
+    // Q operand: Q[qrow][16 c + 4 lg + e].
+    float4 qf[NC];
     {
-        const float* qp = a.q + (static_cast<int64_t>(bh) * a.rows + (row_ok ? qrow : 0)) * D + 16 * lg;
+        const float* qp = a.q + (static_cast<int64_t>(bh) * a.rows + (row_ok ? qrow : 0)) * D + 4 * lg;
 #pragma unroll
-        for (int h = 0; h < H; ++h)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                qf[h][c] = row_ok ? *reinterpret_cast<const float4*>(qp + 64 * h + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int c = 0; c < NC; ++c)
+            qf[c] = row_ok ? *reinterpret_cast<const float4*>(qp + 16 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    // keys < wg_end reach some row of the tile
-    const int wg_end = a.causal ? min(p0 + min(r0 + QR, a.rows), n_keys) : n_keys;
-    const float* kb = a.k + static_cast<int64_t>(bkv) * a.keys * D;
-    const float* vb = a.v + static_cast<int64_t>(bkv) * a.keys * D;
+    const float* kb = a.k + static_cast<int64_t>(bkv) * a.keys * D + 4 * lg;
+    const float* vb = a.v + static_cast<int64_t>(bkv) * a.keys * D + 4 * lr;
     f32x4 acc[4 * H];   // O[row 4 lg + e][dim 64 (db / 4) + 4 lr + db % 4]
 #pragma unroll
     for (int db = 0; db < 4 * H; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.0f;   // statistics of row lr of this wave
 
-    // K/V steps pass through registers one step ahead: the next step's
-    // loads are issued as soon as the current one is in LDS, so they are in
-    // flight during its scores and p . V.
-    constexpr int kU = ST * D / 4 / kThreads;   // float4s of K (and of V) per thread per step
-    float4 nk_reg[kU], nv_reg[kU];
-    auto load_step = [&](int t0) {
-        const int nkt = min(ST, n_keys - t0);
+    struct Block {
+        float4 k[NB][NC];   // K[k0 + 16 nb + lr][16 c + 4 lg ..]
+        float4 v[NS][H];    // V[k0 + 16 (s / 4) + 4 lg + s % 4][64 h + 4 lr ..]
+    };
+    // Keys past the end read the last one; they are masked.
+    auto load = [&](int k0, Block& b) {
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int e = tid + u * kThreads;
-            const int j = e / (D / 4), c = e - j * (D / 4);
-            nk_reg[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            nv_reg[u] = nk_reg[u];
-            if (j < nkt) {
-                nk_reg[u] = *reinterpret_cast<const float4*>(kb + static_cast<int64_t>(t0 + j) * D + 4 * c);
-                nv_reg[u] = *reinterpret_cast<const float4*>(vb + static_cast<int64_t>(t0 + j) * D + 4 * c);
-            }
+        for (int nb = 0; nb < NB; ++nb) {
+            const float* p = kb + static_cast<int64_t>(min(k0 + 16 * nb + lr, n_keys - 1)) * D;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) b.k[nb][c] = *reinterpret_cast<const float4*>(p + 16 * c);
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const float* p = vb + static_cast<int64_t>(min(k0 + 16 * (s / 4) + 4 * lg + s % 4, n_keys - 1)) * D;
+#pragma unroll
+            for (int h = 0; h < H; ++h) b.v[s][h] = *reinterpret_cast<const float4*>(p + 64 * h);
         }
     };
-    if (tid < 2) v_special[tid] = 0;
-    if (wg_end > 0) load_step(0);
-    int parity = 0;
-    for (int s0 = 0; s0 < wg_end; s0 += ST, parity ^= 1) {
-        __syncthreads();   // the previous step is consumed
-        bool special = false;
+    auto compute = [&](int k0, const Block& b) {
+        // S^T = K Q^T: per 16-key tile two accumulators in turn.
+        f32x4 st[NB], su[NB];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int e = tid + u * kThreads;
-            const int j = e / (D / 4), c = e - j * (D / 4);
-            *reinterpret_cast<float4*>(sk + j * PITCH + 4 * c) = nk_reg[u];
-            *reinterpret_cast<float4*>(sv + j * PITCH + 4 * c) = nv_reg[u];
-            // x - x is 0 for finite x, NaN otherwise
-            const float4 v = nv_reg[u];
-            const float d = (v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w);
-            special = special || !(d == 0.0f);
+        for (int nb = 0; nb < NB; ++nb) st[nb] = su[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[nb][c].x, qf[c].x, st[nb], 0, 0, 0);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) su[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[nb][c].y, qf[c].y, su[nb], 0, 0, 0);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[nb][c].z, qf[c].z, st[nb], 0, 0, 0);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) su[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[nb][c].w, qf[c].w, su[nb], 0, 0, 0);
         }
-        if (special) v_special[parity] = 1;
-        if (s0 + ST < wg_end) load_step(s0 + ST);
-        __syncthreads();
-        if (tid == 0) v_special[parity ^ 1] = 0;   // the next step sets it after the next barrier
-
-        const int k0 = s0 + kg * kTile;   // this key group's tile
-        // a tile wholly past the wave's last visible key changes nothing
-        if (k0 > wave_last) continue;
-        const float* skt = sk + kg * kTile * PITCH;
-        const float* svt = sv + kg * kTile * PITCH;
-
-        // S^T = K Q^T for the four 16-key blocks.
-        f32x4 st[4];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) st[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int h = 0; h < H; ++h)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                float4 ka[4];
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb)
-                    ka[nb] = *reinterpret_cast<const float4*>(skt + (16 * nb + lr) * PITCH + 64 * h + 16 * lg + 4 * c);
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[nb].x, qf[h][c].x, st[nb], 0, 0, 0);
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[nb].y, qf[h][c].y, st[nb], 0, 0, 0);
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[nb].z, qf[h][c].z, st[nb], 0, 0, 0);
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) st[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[nb].w, qf[h][c].w, st[nb], 0, 0, 0);
-            }
-        // Scale, mask (tiles that some row does not see whole), online softmax
+        // Scale, mask (blocks that some row does not see whole), online softmax
         // of row lr.  A row that has seen nothing but -inf keeps the maximum
         // -inf and exponentiates against 0.
-        const bool masked = k0 + kTile - 1 > wave_first || !row_ok;
+        const bool masked = k0 + KB - 1 > wave_first;
         float mt = -INFINITY;
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                float v = st[nb][e] * a.scale;
+                float v = (st[nb][e] + su[nb][e]) * a.scale;
                 if (masked) v = k0 + 16 * nb + 4 * lg + e <= my_last ? v : -INFINITY;
                 st[nb][e] = v;
                 mt = fmaxf(mt, v);
@@ -189,18 +160,16 @@ __global__ __launch_bounds__(kThreads) void attention_mfma_kernel(const Attentio
         mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
         const float m_new = fmaxf(m_run, mt);
         const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = exp_nonpos(m_run - m_ref);
         float lt = 0.0f;
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 st[nb][e] = exp_nonpos(st[nb][e] - m_ref);
                 lt += st[nb][e];
             }
-        lt += __shfl_xor(lt, 16, 64);
-        lt += __shfl_xor(lt, 32, 64);
-        const float alpha = exp_nonpos(m_run - m_ref);
-        l_run = l_run * alpha + lt;
+        l_run = fmaf(l_run, alpha, lt);   // (this lane's keys; summed over the lane groups at the end)
         m_run = m_new;
         // Rescale the output rows 4 lg + e by their rows' factors.
 #pragma unroll
@@ -210,54 +179,80 @@ __global__ __launch_bounds__(kThreads) void attention_mfma_kernel(const Attentio
             for (int db = 0; db < 4 * H; ++db) acc[db][e] *= ae;
         }
         // O += P V.  A masked key's zero would turn an infinity or NaN of its
-        // V into NaN: a partly masked tile of a step with such values
-        // multiplies them as 0 and adds them for the rows that see them below.
-        const bool careful = v_special[parity] != 0 && k0 + kTile - 1 > wave_first;
+        // V into NaN: in a partly masked block such values are multiplied as
+        // 0 and added for the rows that see them.
+        bool special = false;
+        if (masked) {
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            const float* vrow = svt + (16 * (s / 4) + 4 * lg + s % 4) * PITCH + 4 * lr;
+            for (int s = 0; s < NS; ++s)
 #pragma unroll
-            for (int h = 0; h < H; ++h) {
-                float4 bv = *reinterpret_cast<const float4*>(vrow + 64 * h);
-                if (careful) {
-                    bv.x = bv.x - bv.x == 0.0f ? bv.x : 0.0f;
-                    bv.y = bv.y - bv.y == 0.0f ? bv.y : 0.0f;
-                    bv.z = bv.z - bv.z == 0.0f ? bv.z : 0.0f;
-                    bv.w = bv.w - bv.w == 0.0f ? bv.w : 0.0f;
+                for (int h = 0; h < H; ++h) {
+                    const float4 v = b.v[s][h];   // x - x is 0 for finite x, NaN otherwise
+                    special = special || !((v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w) == 0.0f);
                 }
-                const float p = st[s / 4][s % 4];
-                acc[4 * h + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, bv.x, acc[4 * h + 0], 0, 0, 0);
-                acc[4 * h + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, bv.y, acc[4 * h + 1], 0, 0, 0);
-                acc[4 * h + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, bv.z, acc[4 * h + 2], 0, 0, 0);
-                acc[4 * h + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, bv.w, acc[4 * h + 3], 0, 0, 0);
-            }
+            special = __any(special);
         }
-        if (careful) {
-            for (int g = 0; g < 4; ++g)
+        if (!special) {
 #pragma unroll
-                for (int s = 0; s < 16; ++s) {
-                    const int key = 16 * (s / 4) + 4 * g + s % 4;
+            for (int s = 0; s < NS; ++s)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int row = r0 + 16 * wr + 4 * lg + e;
-                        const float p = __shfl(st[s / 4][s % 4], 16 * g + 4 * lg + e, 64);
-                        const bool sees = row < a.rows && k0 + key < n_keys && (!a.causal || k0 + key <= p0 + row);
+                for (int h = 0; h < H; ++h) {
+                    const float p = st[s / 4][s % 4];
+                    acc[4 * h + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, b.v[s][h].x, acc[4 * h + 0], 0, 0, 0);
+                    acc[4 * h + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, b.v[s][h].y, acc[4 * h + 1], 0, 0, 0);
+                    acc[4 * h + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, b.v[s][h].z, acc[4 * h + 2], 0, 0, 0);
+                    acc[4 * h + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, b.v[s][h].w, acc[4 * h + 3], 0, 0, 0);
+                }
+        } else {
 #pragma unroll
-                        for (int db = 0; db < 4 * H; ++db) {
-                            const float v = svt[key * PITCH + 64 * (db / 4) + 4 * lr + db % 4];
-                            if (sees && !(v - v == 0.0f)) acc[db][e] = fmaf(p, v, acc[db][e]);
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const float p = st[s / 4][s % 4];
+                    const float v[4] = {b.v[s][h].x, b.v[s][h].y, b.v[s][h].z, b.v[s][h].w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        acc[4 * h + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, v[i] - v[i] == 0.0f ? v[i] : 0.0f,
+                                                                              acc[4 * h + i], 0, 0, 0);
+                        for (int g = 0; g < 4; ++g) {
+                            const int key = k0 + 16 * (s / 4) + 4 * g + s % 4;
+                            const float vk = __shfl(v[i], lr + 16 * g, 64);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int row = r0 + 16 * wr + 4 * lg + e;
+                                const float pk = __shfl(p, 4 * lg + e + 16 * g, 64);
+                                const bool sees = row < a.rows && key < n_keys && (!a.causal || key <= p0 + row);
+                                if (sees && !(vk - vk == 0.0f)) acc[4 * h + i][e] = fmaf(pk, vk, acc[4 * h + i][e]);
+                            }
                         }
                     }
                 }
         }
+    };
+
+    Block b0, b1;
+    int k0 = kg * KB;
+    if (k0 <= wave_last) {
+        load(k0, b0);
+        while (true) {
+            load(k0 + KS * KB, b1);
+            compute(k0, b0);
+            k0 += KS * KB;
+            if (k0 > wave_last) break;
+            load(k0 + KS * KB, b0);
+            compute(k0, b1);
+            k0 += KS * KB;
+            if (k0 > wave_last) break;
+        }
     }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
 
     // Merge the key groups' triples into group 0 (fixed order: group 0, 1,
     // ..): m = max m_g, l = sum l_g e^(m_g - m), O = sum O_g e^(m_g - m).
-    if constexpr (KS > 1) {
-        __syncthreads();   // every wave is past its last LDS read
-        float* so = sk;                         // [KS - 1][RW][16 rows][D]
-        float* sst = sv;                        // [KS - 1][RW][16 rows][2]
+    {
+        __shared__ __align__(16) float so[(KS - 1) * RW * 16 * D];   // [KS - 1][RW][16 rows][D]
+        __shared__ float sst[(KS - 1) * RW * 16 * 2];                // [KS - 1][RW][16 rows][2]
         if (kg > 0) {
             float* o = so + ((kg - 1) * RW + wr) * 16 * D;
 #pragma unroll
@@ -330,36 +325,26 @@ __global__ __launch_bounds__(kThreads) void attention_mfma_kernel(const Attentio
 
 template <int D, int RW, int KS>
 int launch(const AttentionCall& c, const char* op, hipStream_t stream) {
-    constexpr int kLds = 2 * kTile * KS * (D + 4) * 4;
-    auto kernel = attention_mfma_kernel<D, RW, KS>;
-    // (above the 64 KB default; a refused attribute fails the launch)
-    static const hipError_t lds_set = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-    if (lds_set != hipSuccess) return fail_hip(lds_set, op);
     const int64_t grid = static_cast<int64_t>((c.rows + 16 * RW - 1) / (16 * RW)) * c.batch * c.heads;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), kLds, stream, c);
+    const int cus = cu_count();
+    const int fold = c.causal && grid > cus && grid <= 2 * cus ? cus : 0;
+    hipLaunchKernelGGL((attention_mfma_kernel<D, RW, KS>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, stream, c,
+                       fold);
     return check_launch(op, stream);
 }
 
-// Key groups per workgroup (64 / groups query rows each), from sweeps on
-// MI355X: one when a single tile holds the keys, or when one-group workgroups
-// already number more than 512 (1000 x 1500, 64 heads of 128: 408 us, two
-// groups 514); four when even 16-row tiles would leave compute units idle and
-// the keys are many (16 x 2000, 8 heads of 64: 43 us, two groups 65, one 107;
-// head_dim 128 lacks the LDS); two otherwise (512 x 512, 15 heads: 20.5 us,
-// one group 31, four 23).  A cache's key count is on the device: its rows
-// stand for it.  VELOMIND_ATTN_SPLIT = 1 or 2 overrides (sweeps).
+// Key groups per workgroup (64 / groups query rows each): four, which cut the
+// last rows' chain of blocks the most, while the 16-row tiles are few enough
+// that chains and not throughput bound the call, else two (sharing K and V
+// lines in L1 between two row blocks).  MI355X: 512 x 512, 15 heads of 64 (480
+// tiles) 15.5 us against 18.4 with two, 16 x 2000, 8 heads 29 against 53; 512
+// cached rows, 32 heads of 64 (1024 tiles) 27.7 against 22.7, 1500 rows 123
+// against 120; 150 x 498, 128 heads of 128 (1280 tiles) 71 against 84, 1000 x
+// 1500, 64 heads (4032 tiles) 389 against 380.  One group was slower
+// everywhere but on a few keys.
 int key_groups(const AttentionCall& c) {
-    static const int forced = [] {
-        const char* e = std::getenv("VELOMIND_ATTN_SPLIT");
-        const int v = e ? std::atoi(e) : 0;
-        return (v == 1 || v == 2) ? v : 0;
-    }();
-    if (forced) return forced;
-    const int64_t bh = static_cast<int64_t>(c.batch) * c.heads;
-    const int keys = c.pos ? c.rows : c.keys;
-    if ((static_cast<int64_t>(c.rows) + 63) / 64 * bh > 512 || (keys <= kTile && !c.pos)) return 1;
-    return c.head_dim == 64 && (static_cast<int64_t>(c.rows) + 15) / 16 * bh <= 256 && keys > 256 ? 4 : 2;
+    const int64_t tiles = (static_cast<int64_t>(c.rows) + 15) / 16 * c.batch * c.heads;
+    return tiles <= (c.head_dim == 64 ? 512 : 2048) ? 4 : 2;
 }
 
 }  // namespace
@@ -371,11 +356,9 @@ bool attention_mfma_takes(const AttentionCall& c) {
 }
 
 int attention_mfma(const AttentionCall& c, const char* op, hipStream_t stream) {
-    const int groups = key_groups(c);
-    if (c.head_dim == 128)
-        return groups == 1 ? launch<128, 4, 1>(c, op, stream) : launch<128, 2, 2>(c, op, stream);
-    if (groups == 4) return launch<64, 1, 4>(c, op, stream);
-    return groups == 1 ? launch<64, 4, 1>(c, op, stream) : launch<64, 2, 2>(c, op, stream);
+    const bool four = key_groups(c) == 4;
+    if (c.head_dim == 128) return four ? launch<128, 1, 4>(c, op, stream) : launch<128, 2, 2>(c, op, stream);
+    return four ? launch<64, 1, 4>(c, op, stream) : launch<64, 2, 2>(c, op, stream);
 }
 
 }  // namespace vmhip

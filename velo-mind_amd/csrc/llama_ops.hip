@@ -583,9 +583,9 @@ namespace {
 hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
 
 // From here on attention runs on the matrix cores (head_dim 64 or 128): 512 x
-// 512, 15 heads of 64: 20.5 us against 117.6 with a wave per query row; 64 x 64,
-// 32 heads: 6.8 against 8.9; 5 x 700, 8 heads: 18.4 against 37.7.  Below, the
-// tile's padding costs more (13 x 13, 16 heads of 128: 9.4 against 6.0).
+// 512, 15 heads of 64: 15.5 us against 117.6 with a wave per query row; 64 x 64,
+// 32 heads: 6.5 against 8.9; 5 x 700, 8 heads: 13.8 against 37.7.  With fewer
+// rows or keys there is nothing to gain (13 x 13, 16 heads of 128: 6 either way).
 constexpr int64_t kMfmaRows = 5, kMfmaKeys = 48;
 
 constexpr size_t kChainMaxLds = 160 * 1024;   // dynamic LDS of the V-staging attention kernels (no static LDS)
