@@ -126,3 +126,31 @@ def test_half_infinity_and_nan(hip, bf16):
     hip.qmm(da.addr, dt, dq.addr, ds.addr, hip.DTYPE_F32, dc.addr, dt, m, k, n, 1, 0)
     out = _wide(dc.download(np.uint16, (m, n)), bf16)
     assert np.all(np.isposinf(out[1])) and np.all(np.isnan(out[3])) and np.all(np.isfinite(out[[0, 2, 4]]))
+
+
+@pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
+@pytest.mark.parametrize("m,k,n", [(1, 2048, 5633), (4, 5632, 2049), (9, 2048, 515)])
+def test_ragged_first_call_is_captured(hip, kind, block, m, k, n):
+    # a stream whose first call is recorded has no split scratch: such widths
+    # take the kernel that needs none, and every replay gives its result
+    import torch
+
+    rng = np.random.default_rng(m + n)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    da, dq, ds = (torch.from_numpy(np.ascontiguousarray(t)).cuda() for t in (x, q.view(np.int8), s))
+    out = torch.zeros(m, n, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print(f"case captured {kind} m={m} k={k} n={n}", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        hip.qmm_f32(da.data_ptr(), dq.data_ptr(), ds.data_ptr(), out.data_ptr(), m, k, n, qt, block,
+                    stream=stream.cuda_stream)
+    wd = _dense(v, s, block)
+    bound = (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * (np.abs(x.astype(np.float64)) @ np.abs(wd)) + 1e-30
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.all(np.abs(out.cpu().numpy().astype(np.float64) - x.astype(np.float64) @ wd) <= bound)

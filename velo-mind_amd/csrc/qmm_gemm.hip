@@ -364,6 +364,13 @@ constexpr int kHalfRowsDirect = 128;
 int gemm_qmm_half(const uint16_t* a, bool bf16, const uint8_t* wq, const void* scale, bool scale_half, uint16_t* c,
                   int m, int k, int n, int quant_type, int block_size, hipStream_t stream) {
     GemmOperands o{a, 1, nullptr, wq, scale, scale_half, c, m, k, n, block_size, 0};
+    // Scratch that cannot grow during graph capture leaves the call to the
+    // staged fp32 form, whose buffer an earlier call may have sized.
+    const auto refused = [](int rc) {
+        if (rc != VM_HIP_EINVAL) return rc;
+        clear_error();
+        return VM_HIP_EUNSUPPORTED;
+    };
     VM_TRY(gemm_kind(m, k, n, quant_type, block_size, &o.kind));
     const int kp = (k + 31) / 32 * 32;
     const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0;
@@ -372,14 +379,15 @@ int gemm_qmm_half(const uint16_t* a, bool bf16, const uint8_t* wq, const void* s
     // 11.6 us against 13.0, M = 128, 960 x 2560 8.0 against 9.6).
     if (k % 32 != 0 || !aligned || m > kHalfRowsDirect) {
         void* aux = nullptr;
-        VM_TRY(get_aux(stream, a_stage_half_bytes(m, kp, true) / 2, &aux));
+        const int rc = get_aux(stream, a_stage_half_bytes(m, kp, true) / 2, &aux);
+        if (rc != 0) return refused(rc);
         hipLaunchKernelGGL(gemm_prep_half_kernel, dim3((kp / 8 + 7) / 8, (m + 31) / 32), dim3(256), 0, stream, a,
                            static_cast<u32x4*>(aux), m, k, kp, k % 8 == 0 && aligned ? 1 : 0);
         VM_TRY(check_launch("QuantizedMatMul", stream));
         o.a = aux;
         o.layout = 0;
     }
-    return quad_qmm_half(o, bf16, stream);
+    return refused(quad_qmm_half(o, bf16, stream));
 }
 
 }  // namespace vmhip

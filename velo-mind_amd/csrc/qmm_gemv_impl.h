@@ -876,8 +876,11 @@ int launch_cfg(const float* a, const Member* members, int count, int m, int k, i
     const int64_t nblk = KIND == 0 ? 1 : (static_cast<int64_t>(k) + block_size - 1) / block_size;
     GemvMembers mb{};
     int tiles = 0, n_total = 0;
+    bool ragged = false;
     for (int g = 0; g < count; ++g) {
         const int n = members[g].n;
+        ragged = ragged || n % kVec != 0 || reinterpret_cast<uintptr_t>(members[g].wq) % 16 != 0 ||
+                 reinterpret_cast<uintptr_t>(members[g].scale) % 16 != 0;
         mb.wq[g] = members[g].wq;
         mb.scale[g] = members[g].scale;
         mb.c[g] = members[g].c;
@@ -892,8 +895,17 @@ int launch_cfg(const float* a, const Member* members, int count, int m, int k, i
     mb.count = count;
     mb.n_total = n_total;
     Workspace ws{};
-    if (cfg.splits > 1)  // two 32-bit counter slots per pair word
-        VM_TRY(get_workspace(stream, 0, 2 * tree_words(cfg.splits, MR, n_total), &ws));
+    if (cfg.splits > 1) {  // two 32-bit counter slots per pair word
+        const int rc = get_workspace(stream, 0, 2 * tree_words(cfg.splits, MR, n_total), &ws);
+        // Ragged widths and unaligned codes or scales whose scratch is refused
+        // (a fixed region that is too small, a first call during graph
+        // capture) keep the kernels that need none.
+        if (rc == VM_HIP_EINVAL && ragged) {
+            clear_error();
+            return VM_HIP_EUNSUPPORTED;
+        }
+        VM_TRY(rc);
+    }
     unsigned long long* pairs = reinterpret_cast<unsigned long long*>(ws.counters);
     const std::size_t lds = (static_cast<std::size_t>(MR) * cfg.chunks_per_split * kChunkK +
                              static_cast<std::size_t>(W) * MR * kVec * L + 4) * sizeof(float);
