@@ -655,7 +655,8 @@ struct QuadConfig {
 //     more, where their padding adds less than an eighth: each unpacked
 //     column feeds two row tiles (M = 512, 2048 x 11264 50.8 us against 59.7;
 //     blockwise kinds lack the registers: M = 512, 2048 x 5632 INT4 46 us
-//     against 36).
+//     against 36, and with 16-bit A, where they fit one wave per SIMD, 37
+//     against 31, M = 333, 5632 x 2048 bf16 31.7 against 30.4).
 //   * two waves side by side in N, sharing A's lines in L1, where the tiles are
 //     many enough to do with two waves in K: blockwise above 512 rows from 600 tiles
 //     of 32 x 256 (M = 1024, 2048 x 5632 INT4 76.5 -> 65.8 us; M = 512, 2048 x
