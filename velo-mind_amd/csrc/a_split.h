@@ -6,10 +6,11 @@
 // or is all zeros), and written as two fp16 parts, hi = fp16(a 2^x_r) and
 // lo = fp16(a 2^x_r - hi): 22 significant bits of any finite fp32 row.  The
 // parts are stored per 8-group of consecutive k either row-major or in the
-// MFMA kernel's operand order, where a 1 KB piece holds 32 rows x 16 k and position i of an 8-group holds
-// k = i / 2 + 4 (i % 2).  The staged buffer is [hi: mp x k][lo: mp x k]
-// halves, then the m row exponents (int32) at a 256-byte boundary; mp is m
-// rounded up to 32 rows in operand order, m otherwise.
+// MFMA kernel's operand order, where a 1 KB piece holds 32 rows x 16 k and
+// position i of an 8-group holds k = i / 2 + 4 (i % 2).  The staged buffer is
+// [hi: mp x k][lo: mp x k] halves, then the m row exponents (int32) at a
+// 256-byte boundary; mp is m rounded up to 32 rows in operand order, m
+// otherwise.
 #pragma once
 
 #include <hip/hip_runtime.h>
