@@ -237,8 +237,10 @@ int vm_hip_qmm_f32_noalloc(const float* a, const int8_t* wq, const float* scale,
  * (src/cpu/ops/quantized_matmul.cpp:363-367): (a, scale, c) dtypes in
  * {(F32,F32,F32), (F16,F16,F16), (F16,F32,F16), (BF16,BF16,BF16),
  * (BF16,F32,BF16)}.  16-bit activations are multiplied as they are (by codes
- * that are exact in the same type), accumulation is fp32 and half outputs
- * are rounded to nearest even (include/velomind/dtype.h:53-107).
+ * that are exact in the same type), accumulation is fp32 (a bf16 row whose
+ * products or sums leave fp32's range is scaled, so that only the output
+ * itself can overflow) and half outputs are rounded to nearest even
+ * (include/velomind/dtype.h:53-107).
  */
 int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale,
                int scale_dtype, void* c, int c_dtype, int64_t rows_m, int64_t k, int64_t n,

@@ -154,3 +154,44 @@ def test_ragged_first_call_is_captured(hip, kind, block, m, k, n):
         graph.replay()
         torch.cuda.synchronize()
         assert np.all(np.abs(out.cpu().numpy().astype(np.float64) - x.astype(np.float64) @ wd) <= bound)
+
+
+@pytest.mark.parametrize("half_scale", [False, True])
+@pytest.mark.parametrize("kind,block", KINDS)
+@pytest.mark.parametrize("m,k,n", [(1, 2048, 515), (5, 992, 336), (17, 4096, 130), (40, 95, 67), (130, 1000, 132), (200, 2048, 1100)])
+def test_bf16_products_beyond_fp32(hip, half_scale, kind, block, m, k, n):
+    # rows whose products with the codes, or the sums of those, exceed fp32
+    # although the outputs do not; rows of bf16 subnormals; a row that holds
+    # an infinity; a row whose outputs do exceed bf16
+    rng = np.random.default_rng(m + k + n + block)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    wd = _dense(v, s, block)
+    top = np.abs(x.astype(np.float64) @ wd).max(1)   # outputs of a unit row
+    x[0] *= np.float32(1e38 / max(top[0], 4.0))
+    if m > 4:
+        x[1] *= np.float32(2e-39)
+        x[2, 3] = np.inf
+        x[3] = np.where(v[:, 0] * s[0, 0] >= 0, 3e38, -3e38)
+        x[4] *= np.float32(4e37 / max(top[4], 4.0))
+    if m > 5:
+        x[-1] *= np.float32(1e38 / max(top[-1], 4.0))
+    a = _bits(x, True)
+    sb = _bits(s, True) if half_scale else s
+    da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (a, q.view(np.int8), sb, np.zeros((m, n), np.uint16)))
+    print(f"case bf16 large half_scale={half_scale} {kind} block={block} m={m} k={k} n={n}", flush=True)
+    hip.qmm(da.addr, hip.DTYPE_BF16, dq.addr, ds.addr, hip.DTYPE_BF16 if half_scale else hip.DTYPE_F32, dc.addr,
+            hip.DTYPE_BF16, m, k, n, qt, block)
+    out = _wide(dc.download(np.uint16, (m, n)), True).astype(np.float64)
+    wd = _dense(v, _wide(sb, True) if half_scale else s, block)
+    aw = _wide(a, True).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref, mag = aw @ wd, np.abs(aw) @ np.abs(wd)
+        # a result within half an ulp of bf16's largest number may go either way
+        fits, beyond = np.abs(ref) < 3.3e38, np.abs(ref) > 3.45e38
+        bound = 2.0 ** -8 * 1.01 * np.abs(ref) + 2 * k * 2.0 ** -24 * mag + 2.0 ** -133
+        assert np.all(np.abs(out - ref)[fits] <= bound[fits]), np.max((np.abs(out - ref) / bound)[fits])
+    assert fits[0].all() and fits[-1].all()
+    if m > 4:
+        assert fits[1].all() and not np.isfinite(out[2]).any() and beyond[3].any()
+        assert np.array_equal(out[beyond & np.isfinite(ref)], np.copysign(np.inf, ref[beyond & np.isfinite(ref)]))

@@ -485,17 +485,20 @@ void qmm_quad_kernel(const QuadArgs g) {
         if (left > 3) step(integral_constant<int, 3 % D>{}, kLast);
 
     // ---- epilogue
-    float4 cscale = make_float4(1.f, 1.f, 1.f, 1.f);
-    if constexpr (!C::kBlock) {
-        if constexpr (SH) {
+    auto column_scale = [&]() {
+        if constexpr (C::kBlock) {
+            return make_float4(1.f, 1.f, 1.f, 1.f);
+        } else if constexpr (SH) {
             const auto h = __builtin_amdgcn_raw_buffer_load_b64(srs, static_cast<int>(cs * 2), 0, 0);
-            cscale = make_float4(widen<EL>(h[0]), widen<EL>(h[0] >> 16), widen<EL>(h[1]), widen<EL>(h[1] >> 16));
+            return make_float4(widen<EL>(h[0]), widen<EL>(h[0] >> 16), widen<EL>(h[1]), widen<EL>(h[1] >> 16));
         } else {
-            cscale = __builtin_bit_cast(float4, buffer_load16(srs, static_cast<uint32_t>(cs) * 4u));
+            return __builtin_bit_cast(float4, buffer_load16(srs, static_cast<uint32_t>(cs) * 4u));
         }
-    }
+    };
+    const float4 cscale = column_scale();
     // The outputs of one row: four adjacent columns, or the ones of a moved
     // quad that are the lane's own.
+    bool lost = false;   // bf16: the lane stored an output that is no number
     auto store_row = [&](int row, const float4& v) {
         if (row >= m || col >= n) return;
         const int64_t at = static_cast<int64_t>(row) * n + cs;
@@ -514,6 +517,8 @@ void qmm_quad_kernel(const QuadArgs g) {
             uint16_t h[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) h[j] = EL == EL_BF16 ? f32_to_bf16_ref(e[j]) : f32_to_f16_ref(e[j]);
+            if constexpr (EL == EL_BF16)
+                lost = lost || !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) + fabsf(v.w) <= 3.4028235e38f);
             if (g.c_vec) {   // n % 4 == 0, 8-byte aligned C
                 *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | static_cast<uint32_t>(h[1]) << 16,
                                                           h[2] | static_cast<uint32_t>(h[3]) << 16);
@@ -529,6 +534,8 @@ void qmm_quad_kernel(const QuadArgs g) {
     const __amdgpu_buffer_rsrc_t prs =
         buffer_rsrc(g.partials + static_cast<int64_t>(tile * NW + wn) * splits * (C::kItems * 256), 0x7fffffff);
     constexpr int kOwn = (C::kPhase + C::KW - 1) / C::KW;   // items of a phase that a wave adds up
+    // (unrolled: the results of a phase leave their registers with it)
+#pragma unroll
     for (int ph = 0; ph < C::kItems; ph += C::kPhase) {
         if (ph) __syncthreads();
 #pragma unroll
@@ -569,34 +576,109 @@ void qmm_quad_kernel(const QuadArgs g) {
             }
         }
     }
-    if (splits == 1) return;
-
-    publish_partials();
-    __syncthreads();
-    if (tid == 0) ticket = ticket_take(&g.counters[tile], static_cast<unsigned>(splits));
-    __syncthreads();
-    if (ticket != static_cast<unsigned>(splits - 1)) return;
-    for (int item = wk; item < C::kItems; item += C::KW) {
-        const int row = m0 + (item / M::kElems) * TILE + M::row(item % M::kElems, lg);
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int s0 = 0; s0 < splits; s0 += 4) {
-            u32x4 x[4];
+    if (splits > 1) {
+        publish_partials();
+        __syncthreads();
+        if (tid == 0) ticket = ticket_take(&g.counters[tile], static_cast<unsigned>(splits));
+        __syncthreads();
+        if (ticket != static_cast<unsigned>(splits - 1)) return;
+        for (int item = wk; item < C::kItems; item += C::KW) {
+            const int row = m0 + (item / M::kElems) * TILE + M::row(item % M::kElems, lg);
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int s0 = 0; s0 < splits; s0 += 4) {
+                u32x4 x[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                x[u] = s0 + u < splits && row < m
-                           ? coherent_load16(prs, static_cast<uint32_t>(((s0 + u) * C::kItems + item) * 64 + lane) * 16u)
-                           : u32x4{0u, 0u, 0u, 0u};
+                for (int u = 0; u < 4; ++u)
+                    x[u] = s0 + u < splits && row < m
+                               ? coherent_load16(prs, static_cast<uint32_t>(((s0 + u) * C::kItems + item) * 64 + lane) * 16u)
+                               : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                v.x += __uint_as_float(x[u][0]);
-                v.y += __uint_as_float(x[u][1]);
-                v.z += __uint_as_float(x[u][2]);
-                v.w += __uint_as_float(x[u][3]);
+                for (int u = 0; u < 4; ++u) {
+                    v.x += __uint_as_float(x[u][0]);
+                    v.y += __uint_as_float(x[u][1]);
+                    v.z += __uint_as_float(x[u][2]);
+                    v.w += __uint_as_float(x[u][3]);
+                }
             }
+            store_row(row, v);
         }
-        store_row(row, v);
+        if (tid == 0) __hip_atomic_store(&g.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid == 0) __hip_atomic_store(&g.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+    // bf16 has fp32's range, so products with the codes (16 times them for
+    // INT4) and their sums can leave fp32 although the outputs do not (|a|
+    // from 2.6e36).  Infinities and NaN never turn back into numbers, so an
+    // output that is a number is right; one that is not is summed again by
+    // the lane that stored it, its row scaled as fp32 rows are when they are
+    // staged (a row that itself holds an infinity or NaN stays as it is).
+    // Nothing else pays for it (M = 333, 5632 x 2048 INT4 28.9 us with and
+    // without); a pass over A for its row maxima would cost every call 2 us.
+    if constexpr (EL == EL_BF16) {
+        if (!lost) return;
+        const int groups = g.chunks * (C::kChunk / 8);
+#pragma unroll 1
+        for (int item = 0; item < C::kItems; ++item) {
+            const int owner = splits > 1 ? item % C::KW : item % C::kPhase / kOwn;
+            const int row = m0 + (item / M::kElems) * TILE + M::row(item % M::kElems, lg);
+            if (owner != wk || row >= m) continue;
+            const uint16_t* c = static_cast<const uint16_t*>(g.c) + static_cast<int64_t>(row) * n + cs;
+            bool number = true;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) number = number && (cs + j < col || (c[j] & 0x7F80u) != 0x7F80u);
+            if (number) continue;
+            const uint32_t a_at = AM == AM_PIECES
+                                      ? static_cast<uint32_t>(row / 32) * static_cast<uint32_t>(g.k) * 64u + (row % 32) * 16u
+                                      : static_cast<uint32_t>(row) * static_cast<uint32_t>(g.k) * 2u;
+            constexpr uint32_t kGroupBytes = AM == AM_PIECES ? 512u : 16u;
+            float mx = 0.0f;
+            bool special = false;
+#pragma unroll 1
+            for (int i = 0; i < groups; ++i) {
+                const u32x4 w = buffer_load16(ars, a_at + i * kGroupBytes);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float lo = fabsf(widen<EL>(w[j])), hi = fabsf(widen<EL>(w[j] >> 16));
+                    special = special || !(lo <= 3.4028235e38f) || !(hi <= 3.4028235e38f);
+                    mx = fmaxf(mx, fmaxf(lo, hi));
+                }
+            }
+            if (special) continue;
+            const int x = a_row_exponent(mx);
+            float total[4] = {0.f, 0.f, 0.f, 0.f}, part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int i = 0; i < groups; ++i) {
+                const u32x4 w = buffer_load16(ars, a_at + i * kGroupBytes);
+#pragma unroll
+                for (int kk = 0; kk < 8; ++kk) {
+                    // operand order holds k at position 2 (k % 4) + k / 4
+                    const int p = AM == AM_PIECES ? 2 * (kk % 4) + kk / 4 : kk;
+                    const float av = ldexpf(widen<EL>(w[p / 2] >> (16 * (p % 2))), x);
+                    const uint32_t at = static_cast<uint32_t>(KIND == 2 ? 4 * i + kk / 2 : 8 * i + kk) * un + cs;
+                    const uint32_t codes = buffer_load4(wrs, at);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int b = static_cast<int8_t>(codes >> (8 * j));
+                        const int code = KIND != 2 ? b : kk % 2 ? b >> 4 : static_cast<int8_t>(b << 4) >> 4;
+                        part[j] = fmaf(av, static_cast<float>(code), part[j]);
+                    }
+                }
+                if (C::kBlock && i % 4 == 3) {   // a 32-row chunk
+                    const uint32_t at = static_cast<uint32_t>(i / 4 / g.block_chunks) * un + cs;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float s = SH ? widen<EL>(__builtin_amdgcn_raw_buffer_load_b16(srs, static_cast<int>((at + j) * 2u), 0, 0))
+                                           : __uint_as_float(buffer_load4(srs, (at + j) * 4u));
+                        total[j] = fmaf(part[j], s, total[j]);
+                        part[j] = 0.0f;
+                    }
+                }
+            }
+            const float4 f = column_scale();
+            const float4 v = C::kBlock ? make_float4(total[0], total[1], total[2], total[3])
+                                       : make_float4(part[0] * f.x, part[1] * f.y, part[2] * f.z, part[3] * f.w);
+            store_row(row, make_float4(ldexpf(v.x, -x), ldexpf(v.y, -x), ldexpf(v.z, -x), ldexpf(v.w, -x)));
+        }
+    }
 }
 
 template <int KIND, int TILE, int MT, int W, int NW, int AM, int EL, bool SH, int D>
