@@ -218,14 +218,13 @@ LINEAR_EXACT, LINEAR_DENSE = "exact", "dense"
 
 def split_rows_fp16(x: np.ndarray) -> np.ndarray:
     """The HIP MFMA path's staging of A (rows > 4): row r is scaled by 2^x_r
-    with max|row| * 2^x_r in [2^14, 2^15) (x_r = 0 for an all-zero row or one
-    holding an infinity or NaN) and split into hi = fp16(a * 2^x_r) and
+    with its largest finite magnitude * 2^x_r in [2^14, 2^15) (x_r = 0 where
+    that is zero) and split into hi = fp16(a * 2^x_r) and
     lo = fp16(a * 2^x_r - hi) (fp16 rounding to nearest even, subnormals
     included); returns (hi + lo) * 2^-x_r in float64, the value the MFMAs
     multiply (22 significant bits of each element)."""
     x = np.ascontiguousarray(x, f32)
-    special = ~np.isfinite(x).all(axis=-1)
-    amax = np.where(special, f32(0), np.abs(x).max(axis=-1) if x.shape[-1] else f32(0))
+    amax = np.where(np.isfinite(x), np.abs(x), f32(0)).max(axis=-1) if x.shape[-1] else np.zeros(x.shape[:-1], f32)
     _, e = np.frexp(amax.astype(np.float64))
     xr = np.where(amax > 0, 15 - e, 0).astype(np.int64)
     scaled = np.ldexp(x.astype(np.float64), xr[..., None]).astype(f32)          # exact

@@ -128,6 +128,23 @@ def test_half_infinity_and_nan(hip, bf16):
     assert np.all(np.isposinf(out[1])) and np.all(np.isnan(out[3])) and np.all(np.isfinite(out[[0, 2, 4]]))
 
 
+@pytest.mark.parametrize("m,k,n", [(5, 63, 17), (7, 2048, 515), (40, 96, 64), (6, 8192, 67)])
+def test_fp32_infinity_beside_large_values(hip, m, k, n):
+    # a row's infinity or NaN decides its outputs whatever the row's finite
+    # values are (codes that are never zero), as in the reference's fp32 sums
+    rng = np.random.default_rng(k)
+    q = (rng.integers(1, 128, (k, n)) * rng.choice([-1, 1], (k, n))).astype(np.int8)
+    s = np.full((1, n), 0.01, np.float32)
+    x = (rng.standard_normal((m, k)) * 1e6).astype(np.float32)
+    x[1, 7], x[2, k - 1], x[4, 0] = np.inf, -np.inf, np.nan
+    print(f"case fp32 infinity m={m} k={k} n={n}", flush=True)
+    out = hip.run_qmm(x, q, s, k, 1, 0)
+    inf = np.float32(np.inf)
+    assert np.array_equal(out[1], np.copysign(inf, q[7].astype(np.float32)))
+    assert np.array_equal(out[2], np.copysign(inf, -q[k - 1].astype(np.float32)))
+    assert np.isnan(out[4]).all() and np.isfinite(out[[0, 3]]).all() and np.isfinite(out[5:]).all()
+
+
 @pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
 @pytest.mark.parametrize("m,k,n", [(1, 2048, 5633), (4, 5632, 2049), (9, 2048, 515)])
 def test_ragged_first_call_is_captured(hip, kind, block, m, k, n):

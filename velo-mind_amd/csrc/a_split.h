@@ -2,8 +2,7 @@
 // the kernels that produce them (decode_ops.hip).
 //
 // Row r of A is scaled by 2^x_r, the power of two that puts its largest
-// magnitude in [2^14, 2^15) (x_r = 0 when the row holds an infinity or NaN
-// or is all zeros), and written as two fp16 parts, hi = fp16(a 2^x_r) and
+// finite magnitude in [2^14, 2^15) (x_r = 0 when that is zero), and written as two fp16 parts, hi = fp16(a 2^x_r) and
 // lo = fp16(a 2^x_r - hi): 22 significant bits of any finite fp32 row.  The
 // parts are stored per 8-group of consecutive k either row-major or in the
 // MFMA kernel's operand order, where a 1 KB piece holds 32 rows x 16 k and
@@ -39,7 +38,7 @@ inline std::size_t a_stage_bytes(int64_t m, int64_t k, bool pieces) {
 
 __device__ __forceinline__ int a_row_exponent(float mx) {
     int x = 0;
-    if (mx > 0.0f && mx <= 3.4028235e38f) {
+    if (mx > 0.0f) {
         int e = 0;
         (void)frexpf(mx, &e);   // mx = f * 2^e, f in [0.5, 1)
         x = 15 - e;
@@ -47,15 +46,16 @@ __device__ __forceinline__ int a_row_exponent(float mx) {
     return x;
 }
 
-// Largest magnitude of four values, and whether one is an infinity or NaN.
-__device__ __forceinline__ void a_scan4(const float4& v, float& mx, bool& special) {
-    mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    special = special || !(fabsf(v.x) <= 3.4028235e38f) || !(fabsf(v.y) <= 3.4028235e38f) ||
-              !(fabsf(v.z) <= 3.4028235e38f) || !(fabsf(v.w) <= 3.4028235e38f);
+// Largest finite magnitude of four values.  (Infinities and NaN keep their
+// values whatever the scale; a row's finite values have to stay finite beside
+// them.)
+__device__ __forceinline__ void a_scan4(const float4& v, float& mx) {
+    const float a[4] = {fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, a[i] <= 3.4028235e38f ? a[i] : 0.0f);
 }
 
-// hi / lo of one 8-group; an infinite part (|a| beyond fp16 in an unscaled
-// row) leaves lo at 0.
+// hi / lo of one 8-group; an infinity or NaN leaves lo at 0.
 template <bool PIECES>
 __device__ __forceinline__ void a_split8(const float4& p, const float4& q, int x, half8_t& h, half8_t& l) {
     const float s[8] = {ldexpf(p.x, x), ldexpf(p.y, x), ldexpf(p.z, x), ldexpf(p.w, x),

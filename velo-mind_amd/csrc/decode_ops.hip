@@ -1006,14 +1006,11 @@ __device__ __forceinline__ void stage_rows(float4 (&y)[R][GT][2], int row0, int 
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         mx[r] = 0.0f;
-        bool special = false;
 #pragma unroll
         for (int u = 0; u < GT; ++u) {
-            a_scan4(y[r][u][0], mx[r], special);
-            a_scan4(y[r][u][1], mx[r], special);
+            a_scan4(y[r][u][0], mx[r]);
+            a_scan4(y[r][u][1], mx[r]);
         }
-        // an infinity or NaN anywhere in the row disables the scaling
-        if (special) mx[r] = __builtin_inff();
     }
     block_reduce_rows<R>(mx, part, true);
     half8_t* hi = reinterpret_cast<half8_t*>(ah);

@@ -30,11 +30,11 @@ namespace {
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 
 // A [m, k] fp32 -> two fp16 parts with a power-of-two scale per row: x_r
-// is chosen so that max_k |a[r, k]| * 2^x_r lies in [2^14, 2^15) (x_r = 0
-// for an all-zero row, or one holding an infinity or NaN, which then
-// reaches the output as the reference's fp32 arithmetic would propagate
-// it); hi = fp16(a * 2^x_r) and lo = fp16(a * 2^x_r - hi), the difference
-// being exact in fp32.
+// is chosen so that the largest finite |a[r, k]| * 2^x_r lies in [2^14, 2^15)
+// (x_r = 0 where that is zero; an infinity or NaN goes into hi and reaches
+// the output as the reference's fp32 arithmetic propagates it);
+// hi = fp16(a * 2^x_r) and lo = fp16(a * 2^x_r - hi), the difference being
+// exact in fp32.
 // The parts go out in the operand order of v_mfma_f32_32x32x16_f16, so that one wave's operand for 32 rows and 16 k
 // is 1 KB of consecutive memory: the 16 bytes lane l of the wave loads for
 // row block b (rows 32b .. 32b + 31) and k block q (k 16q .. 16q + 15) --
@@ -77,13 +77,6 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const float* __restrict_
     };
     float4 keep[kSplitHeld][2];
     float mx = 0.0f;
-    bool special = false;
-    auto scan = [&](const float4& x) {
-        const float t = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
-        special |= !(fabsf(x.x) <= 3.4028235e38f) || !(fabsf(x.y) <= 3.4028235e38f) ||
-                   !(fabsf(x.z) <= 3.4028235e38f) || !(fabsf(x.w) <= 3.4028235e38f);
-        mx = fmaxf(mx, t);
-    };
     if (held) {
 #pragma unroll
         for (int r = 0; r < kSplitHeld; ++r) {
@@ -97,19 +90,17 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const float* __restrict_
         }
 #pragma unroll
         for (int r = 0; r < kSplitHeld; ++r) {
-            scan(keep[r][0]);
-            scan(keep[r][1]);
+            a_scan4(keep[r][0], mx);
+            a_scan4(keep[r][1], mx);
         }
     } else {
         for (int g = tid; g < groups; g += 256) {
             float4 p, q;
             load8(g, p, q);
-            scan(p);
-            scan(q);
+            a_scan4(p, mx);
+            a_scan4(q, mx);
         }
     }
-    // an infinity or NaN anywhere in the row disables the scaling
-    if (special) mx = __builtin_inff();
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     if ((tid & 63) == 0) wmax[tid >> 6] = mx;
     __syncthreads();
@@ -161,7 +152,6 @@ __global__ __launch_bounds__(256) void gemm_prep_frag_kernel(const float* __rest
     const int groups = kp >> 3;
     float4 v[R][GT][2];
     float mx[R];
-    bool special[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const float* src = a + static_cast<int64_t>(row0 + r) * k;
@@ -184,18 +174,10 @@ __global__ __launch_bounds__(256) void gemm_prep_frag_kernel(const float* __rest
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         mx[r] = 0.0f;
-        special[r] = false;
 #pragma unroll
         for (int u = 0; u < GT; ++u)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float4 x = v[r][u][h];
-                mx[r] = fmaxf(mx[r], fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
-                special[r] = special[r] || !(fabsf(x.x) <= 3.4028235e38f) || !(fabsf(x.y) <= 3.4028235e38f) ||
-                             !(fabsf(x.z) <= 3.4028235e38f) || !(fabsf(x.w) <= 3.4028235e38f);
-            }
-        // an infinity or NaN anywhere in the row disables the scaling
-        if (special[r]) mx[r] = __builtin_inff();
+            for (int h = 0; h < 2; ++h) a_scan4(v[r][u][h], mx[r]);
         for (int off = 32; off > 0; off >>= 1) mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], off));
     }
     if ((tid & 63) == 0)
