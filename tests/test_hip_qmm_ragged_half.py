@@ -75,6 +75,29 @@ def test_ragged_gemv(hip, kind, block, m, k, n):
         assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= bound)
 
 
+@pytest.mark.parametrize("m", [1, 3])
+@pytest.mark.parametrize("k,n", [(64, 31), (2048, 515), (5632, 2049), (2048, 512)])
+def test_ragged_gemv_large_values(hip, m, k, n):
+    # sums of value times code that fill fp32 (at most 2e38), of either sign;
+    # (512 columns: aligned width, codes at an odd address)
+    rng = np.random.default_rng(k + n)
+    q, s, v, qt = _weights(rng, "int4", 32, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x *= np.float32(2e38 / np.abs((x[:, :k // 32 * 32].reshape(m, -1, 32, 1) * v[:k // 32 * 32].reshape(1, -1, 32, n))
+                                  .cumsum(2)).max())
+    print(f"case ragged gemv large m={m} k={k} n={n}", flush=True)
+    wd = _dense(v, s, 32)
+    shift = 1 if n == 512 else 0
+    buf = np.zeros(q.nbytes + 1, np.int8)
+    buf[shift:shift + q.nbytes] = q.view(np.int8).reshape(-1)
+    da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (x, buf, s, np.zeros((m, n), np.float32)))
+    hip.qmm_f32(da.addr, dq.addr + shift, ds.addr, dc.addr, m, k, n, qt, 32)
+    out, ref = dc.download(np.float32, (m, n)).astype(np.float64), x.astype(np.float64) @ wd
+    fits = np.abs(ref) < 3.4e38
+    assert np.all(np.abs(out - ref)[fits] <= (2 * k * 2.0 ** -24 * 1.01 * (np.abs(x.astype(np.float64)) @ np.abs(wd)))[fits])
+    assert fits.all()
+
+
 def _bits(x, bf16):
     return O.f32_to_bf16_bits(x) if bf16 else O.f32_to_f16_bits(x)
 

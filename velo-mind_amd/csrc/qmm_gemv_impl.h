@@ -132,6 +132,7 @@ struct GemvMembers {
     uint32_t scale_bytes[kMaxMembers];
     int count;
     int n_total;
+    int ragged;   // a member with n % 16 != 0 or unaligned codes or scales
 };
 
 template <class T>
@@ -222,6 +223,10 @@ __device__ __forceinline__ void gemv_body(
     const uint32_t code_bytes = pick(mb.code_bytes, member);
     const uint32_t scale_bytes = pick(mb.scale_bytes, member);
     const int n_total = GROUPED ? mb.n_total : n;
+    // INT4 sums carry 16 * code.  The factor goes out with the result, or
+    // (ragged members, whose other kernel multiplies by the codes themselves
+    // and so holds four powers of two more) with the staged activations.
+    const float code_unit = mb.ragged ? 1.0f : 0.0625f;
     const int split = blockIdx.y;
     const int splits = gridDim.y;
     // The lane's columns; a group that would cross the row's end (n % 16) moves
@@ -480,6 +485,11 @@ __device__ __forceinline__ void gemv_body(
                         for (int c = 0; c < 4; ++c)
                             t[u][c] = __float_as_uint((__uint_as_float(t[u][c]) * ir) * __uint_as_float(tu[u][c]));
                     }
+                if (CS::kInt4 && mb.ragged)
+#pragma unroll
+                    for (int u = 0; u < kStageBatch; ++u)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) t[u][c] = __float_as_uint(__uint_as_float(t[u][c]) * 0.0625f);
                 // Unconditional writes (surplus ones go to a spare LDS slot)
                 // keep the compiler from sinking loads into per-write branches.
 #pragma unroll
@@ -526,6 +536,9 @@ __device__ __forceinline__ void gemv_body(
 #pragma unroll
                     for (int u = 0; u < kStageBatch; ++u)
                         t[u] = __float_as_uint((__uint_as_float(t[u]) * inv_of(row[u])) * __uint_as_float(tu[u]));
+                if (CS::kInt4 && mb.ragged)
+#pragma unroll
+                    for (int u = 0; u < kStageBatch; ++u) t[u] = __float_as_uint(__uint_as_float(t[u]) * 0.0625f);
 #pragma unroll
                 for (int u = 0; u < kStageBatch; ++u) {
                     const int e = e0 + u * T;
@@ -614,7 +627,7 @@ __device__ __forceinline__ void gemv_body(
                 float v = 0.0f;
 #pragma unroll
                 for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + red_col(cc)];
-                if constexpr (CS::kInt4) v *= 0.0625f;  // INT4 sums carry 16 * code
+                if constexpr (CS::kInt4) v *= code_unit;
                 if constexpr (KIND == 0) v *= scale[col];
                 if constexpr (FX)
                     if (fx.addend) v = fx.addend[static_cast<int64_t>(i) * n + col] + v;
@@ -643,7 +656,7 @@ __device__ __forceinline__ void gemv_body(
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < W; ++w) v += red[(w * MR + i) * kTileCols + red_col(cc)];
-        if constexpr (CS::kInt4) v *= 0.0625f;
+        if constexpr (CS::kInt4) v *= code_unit;
         bool last = true;
         int64_t level_base = 0;
         for (int lvl = 0; (1 << lvl) < splits; ++lvl) {
@@ -894,6 +907,7 @@ int launch_cfg(const float* a, const Member* members, int count, int m, int k, i
     }
     mb.count = count;
     mb.n_total = n_total;
+    mb.ragged = ragged ? 1 : 0;
     Workspace ws{};
     if (cfg.splits > 1) {  // two 32-bit counter slots per pair word
         const int rc = get_workspace(stream, 0, 2 * tree_words(cfg.splits, MR, n_total), &ws);
