@@ -134,6 +134,28 @@ def test_half(hip, bf16, half_scale, kind, block, m, k, n):
     assert np.all(np.abs(out - ref)[fits] <= bound[fits]), np.max((np.abs(out - ref) / bound)[fits])
 
 
+@pytest.mark.parametrize("m,k,n", [(65537 * 32 + 5, 33, 16), (5, 65537 * 64 + 9, 16)])
+def test_half_staging_of_many_blocks(hip, m, k, n):
+    # more than 65535 blocks of 32 rows, or of 64 columns, are staged
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m % 1000)
+    a = torch.randn(m, k, generator=g, device="cuda", dtype=torch.float16)
+    q = torch.randint(-127, 128, (k, n), generator=g, device="cuda", dtype=torch.int8)
+    s = torch.full((1, n), 1e-3, device="cuda")
+    out = torch.zeros(m, n, device="cuda", dtype=torch.float16)
+    print(f"case half staging m={m} k={k} n={n}", flush=True)
+    hip.qmm(a.data_ptr(), hip.DTYPE_F16, q.data_ptr(), s.data_ptr(), hip.DTYPE_F32, out.data_ptr(), hip.DTYPE_F16, m, k, n,
+            1, 0)
+    rows = torch.tensor(sorted({0, 1, min(m, 31), m // 2, max(m - 6, 0), m - 1} & set(range(m))), device="cuda")
+    aw = a[rows].double()
+    ref, mag = aw @ q.double() * 1e-3, aw.abs() @ q.double().abs() * 1e-3
+    # (a sum is in many parts: no chain of additions is longer than 2^16)
+    bound = 2.0 ** -11 * 1.01 * ref.abs() + 2 * min(k, 2 ** 16) * 2.0 ** -24 * mag + 2.0 ** -24
+    assert torch.all((out[rows].double() - ref).abs() <= bound)
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_half_infinity_and_nan(hip, bf16):
     # 5 x 64 times 64 x 32 codes that are never zero: a row's infinity reaches

@@ -214,14 +214,17 @@ __global__ __launch_bounds__(256) void gemm_prep_frag_kernel(const float* __rest
 }
 
 // fp16 or bf16 rows [m, k] to operand order as they are (a copy, zeros past
-// k): workgroup (block of 32 rows, 8 8-groups), thread (row, 8-group).
+// k): workgroup (block of 32 rows, 8 8-groups), thread (row, 8-group), in a
+// one-dimensional grid (at most 2^18 workgroups by gemm_kind's limits, where
+// either count alone can pass the 65535 of grid y).
 // Threads of one 8-group write 512 consecutive bytes; a row's eight groups
 // are one 128-byte read.
 __global__ __launch_bounds__(256) void gemm_prep_half_kernel(const uint16_t* __restrict__ a, u32x4* __restrict__ out,
                                                              int m, int k, int kp, int vec) {
     __shared__ u32x4 tile[32][9];
-    const int g0 = static_cast<int>(blockIdx.x) * 8;
-    const int row0 = static_cast<int>(blockIdx.y) * 32;
+    const unsigned g_blocks = (static_cast<unsigned>(kp) / 8 + 7) / 8;
+    const int g0 = static_cast<int>(blockIdx.x % g_blocks) * 8;
+    const int row0 = static_cast<int>(blockIdx.x / g_blocks) * 32;
     {
         const int r = threadIdx.x / 8, g = threadIdx.x % 8;
         const int c = 8 * (g0 + g);
@@ -363,7 +366,7 @@ int gemm_qmm_half(const uint16_t* a, bool bf16, const uint8_t* wq, const void* s
         void* aux = nullptr;
         const int rc = get_aux(stream, a_stage_half_bytes(m, kp, true) / 2, &aux);
         if (rc != 0) return refused(rc);
-        hipLaunchKernelGGL(gemm_prep_half_kernel, dim3((kp / 8 + 7) / 8, (m + 31) / 32), dim3(256), 0, stream, a,
+        hipLaunchKernelGGL(gemm_prep_half_kernel, dim3((kp / 8 + 7) / 8 * ((m + 31) / 32)), dim3(256), 0, stream, a,
                            static_cast<u32x4*>(aux), m, k, kp, k % 8 == 0 && aligned ? 1 : 0);
         VM_TRY(check_launch("QuantizedMatMul", stream));
         o.a = aux;
