@@ -129,3 +129,23 @@ def test_pack_rejects_odd_int4_block(hip):
     with pytest.raises(hip.VmHipError) as e:
         hip.pack_int4(w.addr, w.addr, w.addr, 4, 4, 3)
     assert e.value.status == hip.EINVAL and "even" in str(e.value)
+
+
+@pytest.mark.parametrize("rows,cols", [(200, 1028), (333, 515)])
+def test_int8_without_scratch_memory(hip, monkeypatch, rows, cols):
+    # device memory that runs out for the column maxima of the two passes
+    # leaves the single pass, which needs none
+    import torch
+
+    w = _normal(rows, cols, rows)
+    d = torch.from_numpy(w).cuda()
+    q = torch.zeros(rows, cols, device="cuda", dtype=torch.int8)
+    s = torch.zeros(cols, device="cuda")
+    stream = torch.cuda.Stream()   # a new stream: no scratch yet
+    torch.cuda.synchronize()
+    monkeypatch.setenv("VELOMIND_FAIL_BACKEND", "HIP:Scratch:allocate")
+    hip.pack_int8(d.data_ptr(), q.data_ptr(), s.data_ptr(), rows, cols, stream=stream.cuda_stream)
+    monkeypatch.delenv("VELOMIND_FAIL_BACKEND")
+    torch.cuda.synchronize()
+    q_ref, s_ref = O.quantize_int8(w)
+    assert np.array_equal(q.cpu().numpy(), q_ref) and np.array_equal(s.cpu().numpy(), s_ref.reshape(-1))

@@ -257,3 +257,32 @@ def test_bf16_products_beyond_fp32(hip, half_scale, kind, block, m, k, n):
     if m > 4:
         assert fits[1].all() and not np.isfinite(out[2]).any() and beyond[3].any()
         assert np.array_equal(out[beyond & np.isfinite(ref)], np.copysign(np.inf, ref[beyond & np.isfinite(ref)]))
+
+
+@pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
+@pytest.mark.parametrize("m,k,n", [(1, 2048, 5633), (4, 5632, 2049), (9, 2048, 515)])
+def test_ragged_without_scratch_memory(hip, monkeypatch, kind, block, m, k, n):
+    # device memory that runs out for a ragged call's scratch leaves the kernel
+    # that needs none; an aligned call reports it
+    import torch
+
+    rng = np.random.default_rng(m + n)
+    q, s, v, qt = _weights(rng, kind, block, k, n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    da, dq, ds = (torch.from_numpy(np.ascontiguousarray(t)).cuda() for t in (x, q.view(np.int8), s))
+    out = torch.zeros(m, n, device="cuda")
+    stream = torch.cuda.Stream()   # a new stream: no scratch yet
+    torch.cuda.synchronize()
+    monkeypatch.setenv("VELOMIND_FAIL_BACKEND", "HIP:Scratch:allocate")
+    print(f"case no memory {kind} m={m} k={k} n={n}", flush=True)
+    hip.qmm_f32(da.data_ptr(), dq.data_ptr(), ds.data_ptr(), out.data_ptr(), m, k, n, qt, block,
+                stream=stream.cuda_stream)
+    if m == 9:
+        with pytest.raises(Exception):
+            hip.qmm_f32(da.data_ptr(), dq.data_ptr(), ds.data_ptr(), out.data_ptr(), m, k, 512, qt, block,
+                        stream=stream.cuda_stream)
+    monkeypatch.delenv("VELOMIND_FAIL_BACKEND")
+    torch.cuda.synchronize()
+    wd = _dense(v, s, block)
+    bound = (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * (np.abs(x.astype(np.float64)) @ np.abs(wd)) + 1e-30
+    assert np.all(np.abs(out.cpu().numpy().astype(np.float64) - x.astype(np.float64) @ wd) <= bound)

@@ -310,16 +310,12 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
     VM_TRY(gemm_kind(m, k, n, quant_type, block_size, &plan.kind));
     const int kp = (k + 31) / 32 * 32;
     const std::size_t bytes = a_stage_bytes(m, kp, true);
-    // A ragged shape whose scratch is refused (a fixed region that is too
-    // small, a buffer that cannot grow during graph capture) keeps the generic
-    // kernel, which needs none.
+    // A ragged shape whose scratch is refused keeps the generic kernel, which
+    // needs none.
     const bool ragged = k % 32 != 0 || n % 16 != 0;
     void* aux = nullptr;
     int rc = get_aux(stream, bytes, &aux);
-    if (rc == VM_HIP_EINVAL && ragged) {
-        clear_error();
-        return VM_HIP_EUNSUPPORTED;
-    }
+    if (ragged && scratch_refused(rc)) return VM_HIP_EUNSUPPORTED;
     VM_TRY(rc);
     auto* ah = static_cast<_Float16*>(aux);
     auto* row_exp = reinterpret_cast<int*>(static_cast<char*>(aux) + a_stage_half_bytes(m, kp, true));
@@ -337,11 +333,7 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
         hipLaunchKernelGGL(gemm_prep_kernel, dim3(m), dim3(256), 0, stream, a, ah, row_exp, m, k, kp, vec);
     VM_TRY(check_launch("QuantizedMatMul", stream));
     rc = gemm_qmm_staged_f32(plan, ah, row_exp, wq, scale, c, m, k, n, block_size, stream);
-    if (rc == VM_HIP_EINVAL && ragged) {
-        clear_error();
-        return VM_HIP_EUNSUPPORTED;
-    }
-    return rc;
+    return ragged && scratch_refused(rc) ? VM_HIP_EUNSUPPORTED : rc;
 }
 
 constexpr int kHalfRowsDirect = 128;
@@ -351,11 +343,7 @@ int gemm_qmm_half(const uint16_t* a, bool bf16, const uint8_t* wq, const void* s
     GemmOperands o{a, 1, nullptr, wq, scale, scale_half, c, m, k, n, block_size, 0};
     // Scratch that cannot grow during graph capture leaves the call to the
     // staged fp32 form, whose buffer an earlier call may have sized.
-    const auto refused = [](int rc) {
-        if (rc != VM_HIP_EINVAL) return rc;
-        clear_error();
-        return VM_HIP_EUNSUPPORTED;
-    };
+    const auto refused = [](int rc) { return scratch_refused(rc) ? VM_HIP_EUNSUPPORTED : rc; };
     VM_TRY(gemm_kind(m, k, n, quant_type, block_size, &o.kind));
     const int kp = (k + 31) / 32 * 32;
     const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0;

@@ -912,12 +912,8 @@ int launch_cfg(const float* a, const Member* members, int count, int m, int k, i
     if (cfg.splits > 1) {  // two 32-bit counter slots per pair word
         const int rc = get_workspace(stream, 0, 2 * tree_words(cfg.splits, MR, n_total), &ws);
         // Ragged widths and unaligned codes or scales whose scratch is refused
-        // (a fixed region that is too small, a first call during graph
-        // capture) keep the kernels that need none.
-        if (rc == VM_HIP_EINVAL && ragged) {
-            clear_error();
-            return VM_HIP_EUNSUPPORTED;
-        }
+        // keep the kernels that need none.
+        if (ragged && scratch_refused(rc)) return VM_HIP_EUNSUPPORTED;
         VM_TRY(rc);
     }
     unsigned long long* pairs = reinterpret_cast<unsigned long long*>(ws.counters);

@@ -353,7 +353,8 @@ int vm_hip_pack_int8(const float* w, int8_t* q, float* scale, int64_t rows, int6
     auto s = static_cast<hipStream_t>(stream);
     // Two passes for matrices wide and tall enough to fill the GPU, when the
     // stream is not being captured (the row partials use the stream's
-    // workspace, sized here) and the second pass's grid holds the rows.
+    // workspace, sized here; refused memory leaves the single pass, which
+    // needs none) and the second pass's grid holds the rows.
     const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(q) % 4 == 0;
     const int64_t row_groups = (rows + 4 * kPackRows - 1) / (4 * kPackRows);
@@ -366,19 +367,22 @@ int vm_hip_pack_int8(const float* w, int8_t* q, float* scale, int64_t rows, int6
         const int64_t rpc = (row_groups + chunks - 1) / chunks * (4 * kPackRows);
         chunks = (rows + rpc - 1) / rpc;
         Workspace ws{};
-        VM_TRY(get_workspace(s, static_cast<std::size_t>(chunks * cols), 0, &ws));
-        const dim3 grid(static_cast<unsigned>(col_groups), static_cast<unsigned>(chunks));
-        const dim3 grid2(static_cast<unsigned>(col_groups), static_cast<unsigned>(row_groups));
-        if (vec) {
-            hipLaunchKernelGGL(pack_int8_colmax_kernel<4>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
-            hipLaunchKernelGGL(pack_int8_quantize_kernel<4>, grid2, dim3(256), 0, s, w, ws.partials,
-                               static_cast<int>(chunks), q, scale, rows, cols);
-        } else {
-            hipLaunchKernelGGL(pack_int8_colmax_kernel<1>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
-            hipLaunchKernelGGL(pack_int8_quantize_kernel<1>, grid2, dim3(256), 0, s, w, ws.partials,
-                               static_cast<int>(chunks), q, scale, rows, cols);
+        const int rc = get_workspace(s, static_cast<std::size_t>(chunks * cols), 0, &ws);
+        if (rc != 0 && !scratch_refused(rc)) return rc;
+        if (rc == 0) {
+            const dim3 grid(static_cast<unsigned>(col_groups), static_cast<unsigned>(chunks));
+            const dim3 grid2(static_cast<unsigned>(col_groups), static_cast<unsigned>(row_groups));
+            if (vec) {
+                hipLaunchKernelGGL(pack_int8_colmax_kernel<4>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
+                hipLaunchKernelGGL(pack_int8_quantize_kernel<4>, grid2, dim3(256), 0, s, w, ws.partials,
+                                   static_cast<int>(chunks), q, scale, rows, cols);
+            } else {
+                hipLaunchKernelGGL(pack_int8_colmax_kernel<1>, grid, dim3(256), 0, s, w, ws.partials, rows, cols, rpc);
+                hipLaunchKernelGGL(pack_int8_quantize_kernel<1>, grid2, dim3(256), 0, s, w, ws.partials,
+                                   static_cast<int>(chunks), q, scale, rows, cols);
+            }
+            return check_launch("QuantizePack", s);
         }
-        return check_launch("QuantizePack", s);
     }
     hipLaunchKernelGGL(pack_int8_kernel, dim3(grid_1d(cols, kColsPerWg)), dim3(kColsPerWg * kRowGroups),
                        0, s, w, q, scale, rows, cols);

@@ -59,6 +59,12 @@ int get_staging(hipStream_t stream, std::size_t bytes, void** out);
 // Grows like the workspace; refused during capture.
 int get_aux(hipStream_t stream, std::size_t bytes, void** out);
 
+// Whether the status of a call whose get_workspace(), get_aux() or
+// get_staging() it may be says that there is no scratch: a fixed region that
+// is too small, growth during graph capture, or device memory that ran out.
+// Clears the error then, for callers that go on with a kernel that needs none.
+bool scratch_refused(int rc);
+
 // While an instance is alive, get_workspace() on this thread hands out the
 // caller's fixed region (counters first, then partials) instead of the
 // per-stream allocation, get_aux() hands out the end of the partials area,

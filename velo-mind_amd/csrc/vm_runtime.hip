@@ -114,6 +114,22 @@ int check_launch(const char* op, hipStream_t stream) {
     return 0;
 }
 
+// hipMalloc of a per-stream buffer; VELOMIND_FAIL_BACKEND="HIP:Scratch:allocate"
+// makes it run out of memory.
+static int scratch_malloc(void** out, std::size_t bytes, const char* what) {
+    *out = nullptr;
+    if (injected_failure("Scratch", "allocate") != 0) return static_cast<int>(hipErrorOutOfMemory);
+    VM_TRY_HIP(hipMalloc(out, bytes), what);
+    return 0;
+}
+
+bool scratch_refused(int rc) {
+    if (rc != VM_HIP_EINVAL && rc != static_cast<int>(hipErrorOutOfMemory)) return false;
+    clear_error();
+    (void)hipGetLastError();   // a failed hipMalloc is not the next launch's error
+    return true;
+}
+
 FixedWorkspaceScope::FixedWorkspaceScope(void* base, std::size_t counter_slots, std::size_t partial_floats,
                                          const char* who)
     : _region{base, counter_slots, partial_floats, who}, _previous(t_fixed) {
@@ -160,7 +176,7 @@ int get_workspace(hipStream_t stream, std::size_t partial_floats, std::size_t co
         }
         const std::size_t counter_bytes = ((cs * sizeof(unsigned)) + 255) & ~std::size_t(255);
         void* base = nullptr;
-        VM_TRY_HIP(hipMalloc(&base, counter_bytes + pf * sizeof(float)), "workspace: hipMalloc");
+        VM_TRY(scratch_malloc(&base, counter_bytes + pf * sizeof(float), "workspace: hipMalloc"));
         // Zero the counters on the stream that will use them: a plain
         // hipMemset runs on the null stream, which is not ordered with the
         // non-blocking streams the kernels are launched on.  (Growth is
@@ -207,7 +223,7 @@ int get_aux(hipStream_t stream, std::size_t bytes, void** out) {
             e.retired.push_back(e.base);
             e.base = nullptr;
         }
-        VM_TRY_HIP(hipMalloc(&e.base, want), "staged A: hipMalloc");
+        VM_TRY(scratch_malloc(&e.base, want, "staged A: hipMalloc"));
         e.bytes = want;
     }
     *out = e.base;
@@ -257,7 +273,7 @@ int get_staging(hipStream_t stream, std::size_t bytes, void** out) {
             e.retired.push_back(e.base);
             e.base = nullptr;
         }
-        VM_TRY_HIP(hipMalloc(&e.base, want), "staging: hipMalloc");
+        VM_TRY(scratch_malloc(&e.base, want, "staging: hipMalloc"));
         e.bytes = want;
     }
     *out = e.base;
