@@ -71,6 +71,13 @@ def test_noalloc_matches_qmm_f32_twice(hip, first, second):
     _check(hip, 12, *second)
 
 
+@pytest.mark.parametrize("m,k,n", [(5, 131072, 32), (20, 147456, 16), (16, 114688, 64)])
+def test_noalloc_takes_few_long_rows(hip, m, k, n):
+    # per-column INT8 rows whose operand-order staging (32 rows) passes the
+    # array's 14 MiB (the last: does not) are staged as they are
+    _check(hip, 41, m, k, n, O.QUANT_INT8)
+
+
 def test_noalloc_on_a_stream_then_null_stream(hip):
     s = hip.Stream()
     try:

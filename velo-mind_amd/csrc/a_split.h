@@ -18,6 +18,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "vm_hip.h"
+
 namespace vmhip {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -35,6 +37,10 @@ inline std::size_t a_stage_half_bytes(int64_t m, int64_t k, bool pieces) {
 inline std::size_t a_stage_bytes(int64_t m, int64_t k, bool pieces) {
     return a_stage_half_bytes(m, k, pieces) + ((static_cast<std::size_t>(m) * 4 + 255) & ~std::size_t(255));
 }
+
+// What the no-allocation entry point's static array holds of staged A and
+// partial tiles together.
+constexpr std::size_t kStaticPartialBytes = VM_HIP_QMM_NOALLOC_SCRATCH_BYTES - VM_HIP_QMM_NOALLOC_COUNTER_BYTES;
 
 __device__ __forceinline__ int a_row_exponent(float mx) {
     int x = 0;

@@ -59,6 +59,8 @@ __device__ __forceinline__ void load8_tail(const float* src, int c, int k, float
     q = make_float4(v[4], v[5], v[6], v[7]);
 }
 
+// PIECES: operand order; else row-major (k a multiple of 32).
+template <bool PIECES>
 __global__ __launch_bounds__(256) void gemm_prep_kernel(const float* __restrict__ a, _Float16* __restrict__ ah,
                                                         int* __restrict__ row_exp, int m, int k, int kp, int vec) {
     __shared__ float wmax[4];
@@ -107,18 +109,15 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const float* __restrict_
     mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     const int x = a_row_exponent(mx);
     if (tid == 0) row_exp[row] = x;
-    const int64_t mp = (static_cast<int64_t>(m) + 31) / 32 * 32;
+    const int64_t mp = PIECES ? (static_cast<int64_t>(m) + 31) / 32 * 32 : m;
     half8v* hi = reinterpret_cast<half8v*>(ah);
     half8v* lo = reinterpret_cast<half8v*>(ah + mp * kp);
-    // 16-byte piece index of the row's 8-group g
-    auto piece = [&](int g) -> int64_t {
-        return (static_cast<int64_t>(row / 32) * (kp / 16) + g / 2) * 64 + row % 32 + 32 * (g % 2);
-    };
     auto split = [&](int g, const float4& p, const float4& q) {
         half8v h, l;
-        a_split8<true>(p, q, x, h, l);
-        hi[piece(g)] = h;
-        lo[piece(g)] = l;
+        a_split8<PIECES>(p, q, x, h, l);
+        const int64_t at = a_piece<PIECES>(row, g, kp);
+        hi[at] = h;
+        lo[at] = l;
     };
     if (held) {
 #pragma unroll
@@ -306,10 +305,14 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
     // Operand order for every shape (it reads faster than rows: M = 16,
     // K = 2048, N = 5632 INT8 9.9 us against 10.8), K padded with zeros.
     GemmPlan plan;
-    plan.pieces = true;
     VM_TRY(gemm_kind(m, k, n, quant_type, block_size, &plan.kind));
     const int kp = (k + 31) / 32 * 32;
-    const std::size_t bytes = a_stage_bytes(m, kp, true);
+    // Few rows so long that operand order's 32 are more than the no-allocation
+    // entry point's array holds: per-column INT8 takes them row by row (in
+    // every entry point, so that all give the same bits).
+    plan.pieces = !(plan.kind == 0 && m <= 32 && k % 32 == 0 && n % 16 == 0 &&
+                    a_stage_bytes(m, kp, true) > kStaticPartialBytes);
+    const std::size_t bytes = a_stage_bytes(m, kp, plan.pieces);
     // A ragged shape whose scratch is refused keeps the generic kernel, which
     // needs none.
     const bool ragged = k % 32 != 0 || n % 16 != 0;
@@ -318,10 +321,13 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
     if (ragged && scratch_refused(rc)) return VM_HIP_EUNSUPPORTED;
     VM_TRY(rc);
     auto* ah = static_cast<_Float16*>(aux);
-    auto* row_exp = reinterpret_cast<int*>(static_cast<char*>(aux) + a_stage_half_bytes(m, kp, true));
+    auto* row_exp = reinterpret_cast<int*>(static_cast<char*>(aux) + a_stage_half_bytes(m, kp, plan.pieces));
     const int vec = k % 32 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 ? 1 : 0;
     const int gt = (kp / 8 + 255) / 256;
     const int rows_per_wg = prep_rows_per_wg(m, gt);
+    if (!plan.pieces) {
+        hipLaunchKernelGGL(gemm_prep_kernel<false>, dim3(m), dim3(256), 0, stream, a, ah, row_exp, m, k, kp, vec);
+    } else
 #define VM_PREP(RX, GX)                                                                                           \
     if (gt == GX && rows_per_wg == RX)                                                                            \
         hipLaunchKernelGGL((gemm_prep_frag_kernel<RX, GX>), dim3((m + RX - 1) / RX), dim3(256), 0, stream, a, ah, \
@@ -330,7 +336,7 @@ int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c
     VM_PREP(8, 1) VM_PREP(4, 1) VM_PREP(2, 1) VM_PREP(1, 1) VM_PREP(4, 2) VM_PREP(2, 2) VM_PREP(1, 2)
     VM_PREP(2, 3) VM_PREP(1, 3)
 #undef VM_PREP
-        hipLaunchKernelGGL(gemm_prep_kernel, dim3(m), dim3(256), 0, stream, a, ah, row_exp, m, k, kp, vec);
+        hipLaunchKernelGGL(gemm_prep_kernel<true>, dim3(m), dim3(256), 0, stream, a, ah, row_exp, m, k, kp, vec);
     VM_TRY(check_launch("QuantizedMatMul", stream));
     rc = gemm_qmm_staged_f32(plan, ah, row_exp, wq, scale, c, m, k, n, block_size, stream);
     return ragged && scratch_refused(rc) ? VM_HIP_EUNSUPPORTED : rc;

@@ -805,7 +805,8 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
 
 template <int KIND, int AM, int EL, bool SH>
 int launch_mode(const GemmOperands& o, hipStream_t s) {
-    const std::size_t a_bytes = AM == AM_PIECES ? a_stage_bytes(o.m, (o.k + 31) / 32 * 32, true) : 0;
+    const std::size_t a_bytes =
+        AM == AM_PIECES || EL == EL_F32 ? a_stage_bytes(o.m, (o.k + 31) / 32 * 32, AM == AM_PIECES) : 0;
     const QuadConfig c = choose_quad<KIND, AM, EL>(o.m, o.k, o.n, a_bytes);
     if (c.tile == 16) {
         if (c.waves == 4) return launch_quad<KIND, 16, 1, 4, 1, AM, EL, SH, 3>(o, c.splits, s);
