@@ -212,3 +212,16 @@ def test_wide_long_k(hip, monkeypatch, kind, block):
     print(f"case wide long-k {forced} kind={kind}", flush=True)
     _check(hip.run_qmm(x, q, s, k, qt, blk), ref)
     monkeypatch.delenv("VELOMIND_GEMM_WIDE")
+
+
+@pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
+@pytest.mark.parametrize("m,n", [(384, 300), (401, 4500), (700, 1100), (1025, 2600)])
+def test_row_panels(hip, kind, block, m, n):
+    # tiles are numbered in panels of about 256 rows, the last one shorter:
+    # every tile of every panel is written
+    k = 96
+    rng = np.random.default_rng(m + n)
+    q, s, qt, blk = _weights(kind, k, n, rng, block)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    print(f"case panels kind={kind} m={m} k={k} n={n}", flush=True)
+    _check(hip.run_qmm(x, q, s, k, qt, blk), O.qmm(x, q.view(np.int8), s, k, O.QUANT_INT4 if qt == 2 else O.QUANT_INT8, blk))

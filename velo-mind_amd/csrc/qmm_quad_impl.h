@@ -196,6 +196,7 @@ struct QuadArgs {
     int chunks;             // of K
     int chunks_per_wave;
     int tiles_n, tiles_m;
+    int panel;              // row tiles of a panel
     uint32_t a_bytes, lo_offset, code_bytes, scale_bytes;
     int c_vec;
 };
@@ -240,17 +241,24 @@ void qmm_quad_kernel(const QuadArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lc = lane % TILE;    // operand row of A, column quad of B
     const int lg = lane / TILE;    // 8-row K group
-    // Grid over (split, tile column, tile row), row fastest; workgroups go to
-    // the 8 XCDs round-robin by id, and renumbering gives each XCD a
-    // contiguous run, so that the workgroups of one L2 share weight columns.
+    // Grid over (split, row panel, tile column, tile row), row fastest;
+    // workgroups go to the 8 XCDs round-robin by id, and renumbering gives each
+    // XCD a contiguous run, so that the workgroups of one L2 share weight
+    // columns and, with panels of about 256 rows, A as well: a run over all rows of a
+    // large A reads it whole from beyond the L2 (2048 rows of 2048 x 2048 INT8
+    // 69.7 us in one panel, 49.3 with 512 rows, 48.1 with 256, 48.5 with 128).
     int lin = blockIdx.x;
     {
         const int full = static_cast<int>(gridDim.x) & ~7;
         if (lin < full) lin = (lin & 7) * (full >> 3) + (lin >> 3);
     }
-    const int tile_y = lin % g.tiles_m;
-    const int tile_x = (lin / g.tiles_m) % g.tiles_n;
     const int split = lin / (g.tiles_n * g.tiles_m);
+    const int in_split = lin - split * g.tiles_n * g.tiles_m;
+    const int panel = in_split / (g.panel * g.tiles_n);
+    const int in_panel = in_split - panel * g.panel * g.tiles_n;
+    const int panel_rows = min(g.panel, g.tiles_m - panel * g.panel);
+    const int tile_x = in_panel / panel_rows;
+    const int tile_y = panel * g.panel + in_panel - tile_x * panel_rows;
     const int splits = static_cast<int>(gridDim.x) / (g.tiles_n * g.tiles_m);
     const int n = g.n, m = g.m;
     const int m0 = tile_y * C::BM;
@@ -701,6 +709,12 @@ int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
     const int units = splits * C::KW;
     g.chunks_per_wave = (g.chunks + units - 1) / units;
     splits = (g.chunks + g.chunks_per_wave * C::KW - 1) / (g.chunks_per_wave * C::KW);
+    // Even panels of about 256 rows, the last no shorter than the others by more
+    // than a tile (333 rows in panels of 256 and 77: 4096 x 5632 INT8 52.6 us
+    // against 51.1).  K splits: one panel, their few tiles' runs are short
+    // already (1024 rows of 8192 x 256 INT8 in four splits 52 us, 61 with panels).
+    const int panels = splits > 1 ? 1 : std::max(1, (o.m + 127) / 256);
+    g.panel = (g.tiles_m + panels - 1) / panels;
     Workspace ws{};
     const std::size_t tiles = static_cast<std::size_t>(g.tiles_n) * g.tiles_m;
     if (splits > 1) VM_TRY(get_workspace(stream, tiles * NW * splits * (C::kItems * 256), tiles, &ws));
@@ -742,8 +756,11 @@ struct QuadConfig {
 //   * two waves side by side in N, sharing A's lines in L1, where the tiles are
 //     many enough to do with two waves in K: blockwise above 512 rows from 600 tiles
 //     of 32 x 256 (M = 1024, 2048 x 5632 INT4 76.5 -> 65.8 us; M = 512, 2048 x
-//     11264 64.1 -> 61 to 66, 2048 x 5632 41 -> 43.5), 64-row tiles from 1200 (M = 1024, 2048 x 11264
-//     INT8 102 -> 95; 704 tiles 51.7 -> 55.7).
+//     11264 64.1 -> 61 to 66, 2048 x 5632 41 -> 43.5); 64-row tiles from 1024
+//     where the wider ones, at two units of time each, take no more rounds of
+//     the GPU (M = 1024, INT8: 1024 tiles of 576 x 8192 31.7 -> 29.8 us, of 2048 x
+//     8192 69.8 -> 68.0; 768 tiles, 2048 rows of 2048 x 3072, would take four
+//     rounds for three, 58.9 -> 63.3; below 1024 tiles either way within 5 %).
 //   * eight waves per tile; four once the tiles alone fill the GPU (more than
 //     260), or when a 16-row tile's K is too short for eight (576 x 1536).
 //   * K splits only where the tiles leave compute units idle: 16-row tiles
@@ -775,7 +792,8 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
         if (KIND == 0 && AM == AM_PIECES && tiles64 >= 170 && (m + 63) / 64 * 64 <= (m + 31) / 32 * 36) {
             c.mt = 2;
             c.waves = 4;
-            c.pair = tiles64 >= 1200;
+            const long cus = 256, rounds = (tiles64 + cus - 1) / cus;
+            c.pair = tiles64 >= 1024 && 2 * ((tiles_of(64, 256) + cus - 1) / cus) <= rounds;
         } else if (KIND != 0 && AM == AM_PIECES && m > 512 && tiles_of(32, 256) >= 600) {
             c.waves = 4;
             c.pair = true;
