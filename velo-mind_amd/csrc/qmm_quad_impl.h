@@ -768,8 +768,10 @@ struct QuadConfig {
 //     about 60 workgroups run, wider tiles up to about 260 workgroups, never
 //     below two chunks a wave (M = 64, 2048 x 2048 INT4: four splits 11.9 us,
 //     one 14); at most six there, at most twelve on 16-row tiles.
-// A call's fp32 partial tiles and staged A stay below 14 MiB, the room that
-// the no-allocation entry point has, so that both choose alike.
+// Where the staged A leaves the no-allocation entry point room in its static
+// array, a call's fp32 partial tiles stay within it, so that all entry points
+// choose alike; it refuses longer A, and takes no 16-bit calls, and these have
+// all their splits (M = 512, 8192 x 512 INT8 33.6 us in four splits, 44.5 in one).
 // VELOMIND_GEMM_WIDE="BM,BN,S,D[,G]" or VELOMIND_GEMM_CFG="BM,BN,S[,D]" force
 // the row tile (nearest to BM), paired waves with BN of 256 or more, S splits
 // and, with D or G of 2, eight waves.
@@ -806,7 +808,9 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
     auto partials = [&](int s) {
         return s > 1 ? static_cast<double>(tiles_of(c.tile * c.mt, 4 * c.tile)) * s * c.tile * c.mt * 4 * c.tile * 4 : 0.0;
     };
-    while (c.splits > 1 && partials(c.splits) + static_cast<double>(a_bytes) > (14 << 20) - 65536) --c.splits;
+    constexpr std::size_t kRoom = kStaticPartialBytes - 65536;
+    if (EL == EL_F32 && a_bytes <= kRoom)
+        while (c.splits > 1 && partials(c.splits) > static_cast<double>(kRoom - a_bytes)) --c.splits;
     int bm = 0, bn = 0, s = 0, d = 0, g = 0;
     const char* env = std::getenv("VELOMIND_GEMM_WIDE");
     int got = env ? std::sscanf(env, "%d,%d,%d,%d,%d", &bm, &bn, &s, &d, &g) : 0;
@@ -823,8 +827,7 @@ QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
 
 template <int KIND, int AM, int EL, bool SH>
 int launch_mode(const GemmOperands& o, hipStream_t s) {
-    const std::size_t a_bytes =
-        AM == AM_PIECES || EL == EL_F32 ? a_stage_bytes(o.m, (o.k + 31) / 32 * 32, AM == AM_PIECES) : 0;
+    const std::size_t a_bytes = EL == EL_F32 ? a_stage_bytes(o.m, (o.k + 31) / 32 * 32, AM == AM_PIECES) : 0;
     const QuadConfig c = choose_quad<KIND, AM, EL>(o.m, o.k, o.n, a_bytes);
     if (c.tile == 16) {
         if (c.waves == 4) return launch_quad<KIND, 16, 1, 4, 1, AM, EL, SH, 3>(o, c.splits, s);
