@@ -38,6 +38,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -244,9 +245,9 @@ void qmm_quad_kernel(const QuadArgs g) {
     // Grid over (split, row panel, tile column, tile row), row fastest;
     // workgroups go to the 8 XCDs round-robin by id, and renumbering gives each
     // XCD a contiguous run, so that the workgroups of one L2 share weight
-    // columns and, with panels of about 256 rows, A as well: a run over all rows of a
+    // columns and, in panels (launch_quad), A as well: a run over all rows of a
     // large A reads it whole from beyond the L2 (2048 rows of 2048 x 2048 INT8
-    // 69.7 us in one panel, 49.3 with 512 rows, 48.1 with 256, 48.5 with 128).
+    // 69.7 us in one panel, 49.3 in panels of 512 rows, 48.1 of 256).
     int lin = blockIdx.x;
     {
         const int full = static_cast<int>(gridDim.x) & ~7;
@@ -709,11 +710,21 @@ int launch_quad(const GemmOperands& o, int splits, hipStream_t stream) {
     const int units = splits * C::KW;
     g.chunks_per_wave = (g.chunks + units - 1) / units;
     splits = (g.chunks + g.chunks_per_wave * C::KW - 1) / (g.chunks_per_wave * C::KW);
-    // Even panels of about 256 rows, the last no shorter than the others by more
-    // than a tile (333 rows in panels of 256 and 77: 4096 x 5632 INT8 52.6 us
-    // against 51.1).  K splits: one panel, their few tiles' runs are short
-    // already (1024 rows of 8192 x 256 INT8 in four splits 52 us, 61 with panels).
-    const int panels = splits > 1 ? 1 : std::max(1, (o.m + 127) / 256);
+    // Row tiles of a panel: of the tiles an XCD works on at a time, up to 32 (one
+    // to a compute unit; counting two measured slower), p rows by 32 / p columns
+    // read p row tiles of A and 32 / p column tiles of codes, least at p = sqrt(32
+    // codes / A).  Panels of equal height, so that the last is not a short one.
+    // One panel to 384 rows (192 rows of 4096 x 5632 INT8 33.7 us, 35.7 in two),
+    // for 16-bit A, half the size (1024 rows of 4096 x 1024 bf16 INT4 24.9, 26.7;
+    // of 2048 x 5632 54.2, 52.5), and for K splits, whose runs are short already
+    // (1024 rows of 8192 x 256 INT8 in four splits 52, 61).
+    int panels = 1;
+    if (EL == EL_F32 && splits == 1 && o.m > 384) {
+        const double tile_codes = C::NT * (KIND == 2 ? 0.5 : 1.0), tile_a = C::BM * 4.0;
+        const double active = std::min(32.0, g.tiles_n * static_cast<double>(g.tiles_m) / 8);
+        const int high = std::max(1, static_cast<int>(std::sqrt(active * tile_codes / tile_a) + 0.5));
+        panels = std::max(1, (g.tiles_m + high / 2) / high);
+    }
     g.panel = (g.tiles_m + panels - 1) / panels;
     Workspace ws{};
     const std::size_t tiles = static_cast<std::size_t>(g.tiles_n) * g.tiles_m;
