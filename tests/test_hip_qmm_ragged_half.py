@@ -134,6 +134,48 @@ def test_half(hip, bf16, half_scale, kind, block, m, k, n):
     assert np.all(np.abs(out - ref)[fits] <= bound[fits]), np.max((np.abs(out - ref) / bound)[fits])
 
 
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("m,k,n", [(1, 8192, 20480), (1, 8192, 18304), (2, 8192, 20480)])
+def test_half_large_matrix(hip, captured, m, k, n):
+    # one bf16 row of an INT4 matrix of 75 MB is widened for the decode GEMV (the
+    # second matrix is just below, the third call has two rows); without memory
+    # for the widened rows, as in a stream's first call when it is captured,
+    # the MFMA kernel takes it
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    a = torch.randn(m, k, generator=g, device="cuda")
+    q = torch.randint(-128, 128, (k // 2, n), generator=g, device="cuda", dtype=torch.int8)
+    s = torch.rand(k // 32, n, generator=g, device="cuda") * 1e-3
+    lo = ((q << 4) >> 4).double()
+    wd = torch.stack([lo, (q >> 4).double()], 1).view(k, n) * s.double().repeat_interleave(32, 0)
+    # up to where value times code fills fp32, not 16 times it
+    a[0] *= 2e38 / (8 * 32 * a[0].abs().max())
+    a = a.to(torch.bfloat16)
+    out = torch.zeros(m, n, device="cuda", dtype=torch.bfloat16)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print(f"case half large m={m} k={k} n={n} captured={captured}", flush=True)
+
+    def call():
+        hip.qmm(a.data_ptr(), hip.DTYPE_BF16, q.data_ptr(), s.data_ptr(), hip.DTYPE_F32, out.data_ptr(), hip.DTYPE_BF16,
+                m, k, n, 2, 32, stream=stream.cuda_stream)
+
+    graph = torch.cuda.CUDAGraph()
+    if captured:
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+    ref = a.double() @ wd
+    bound = 2.0 ** -8 * 1.01 * ref.abs() + 2 * k * 2.0 ** -24 * (a.double().abs() @ wd.abs())
+    for _ in range(2):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay() if captured else call()
+        torch.cuda.synchronize()
+        assert torch.all((out.double() - ref).abs() <= bound)
+
+
 @pytest.mark.parametrize("m,k,n", [(65537 * 32 + 5, 33, 16), (5, 65537 * 64 + 9, 16)])
 def test_half_staging_of_many_blocks(hip, m, k, n):
     # more than 65535 blocks of 32 rows, or of 64 columns, are staged

@@ -58,10 +58,26 @@ __global__ void zero_kernel(float* __restrict__ c, int64_t count) {
 }
 
 __global__ void f32_to_half_kernel(const float* __restrict__ src, uint16_t* __restrict__ dst,
-                                   int64_t count, int is_bf16) {
+                                   int64_t count, int is_bf16, float factor) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= count) return;
-    dst[i] = is_bf16 ? f32_to_bf16_ref(src[i]) : f32_to_f16_ref(src[i]);
+    dst[i] = is_bf16 ? f32_to_bf16_ref(src[i] * factor) : f32_to_f16_ref(src[i] * factor);
+}
+
+// Whether a 16-bit call of a few rows with fp32 scales is widened for the
+// decode GEMV instead of taking the MFMA kernel: the GEMV streams very large
+// matrices better than the conversions cost.  One row, GEMV with conversions
+// against MFMA: bf16 INT4 8192 x 14336 19.7 us, 19.7; 8192 x 20480 28.7, 31.7;
+// 12288 x 49152 76, 89; fp16 INT4 8192 x 28672 31.4, 27.1, 12288 x 49152 78, 82;
+// blockwise INT8 8192 x 28672 47.2, 41.9, 8192 x 57344 91.8, 102; per-column INT8
+// never.  Two rows: INT8 16384 x 16384 52.7, 49.2, 12288 x 49152 128, 136; four:
+// per-column INT8 12288 x 49152 133, 141.  16-bit scales: never (a third
+// conversion).
+bool widen_for_gemv(bool bf16, int64_t m, int64_t k, int64_t n, bool int4, int block_size) {
+    const double codes = (int4 ? 0.5 : 1.0) * static_cast<double>(k) * static_cast<double>(n);
+    if (m == 1) return int4 ? codes >= (bf16 ? 75e6 : 250e6) : block_size > 0 && codes >= 250e6;
+    if (m == 2) return !int4 && codes >= 450e6;
+    return m <= 4 && !int4 && block_size <= 0 && codes >= 550e6;
 }
 
 unsigned blocks_for(int64_t count, int threads) {
@@ -317,16 +333,21 @@ int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale, 
                             static_cast<float*>(c), rows_m, k, n, quant_type, block_size, s);
     if (rows_m == 0 || n == 0) return 0;
 
-    if (k > 0) {
-        const int bs = (quant_type == VM_HIP_QUANT_INT4 && block_size <= 0) ? 32 : block_size;
-        const int rc = gemm_qmm_half(static_cast<const uint16_t*>(a), a_dtype == VM_HIP_DTYPE_BF16,
-                                     reinterpret_cast<const uint8_t*>(wq), scale, scale_dtype != VM_HIP_DTYPE_F32,
-                                     static_cast<uint16_t*>(c), static_cast<int>(rows_m), static_cast<int>(k),
-                                     static_cast<int>(n), quant_type, bs, s);
+    const bool bf16 = a_dtype == VM_HIP_DTYPE_BF16, int4 = quant_type == VM_HIP_QUANT_INT4;
+    const auto direct = [&] {
+        return gemm_qmm_half(static_cast<const uint16_t*>(a), bf16, reinterpret_cast<const uint8_t*>(wq), scale,
+                             scale_dtype != VM_HIP_DTYPE_F32, static_cast<uint16_t*>(c), static_cast<int>(rows_m),
+                             static_cast<int>(k), static_cast<int>(n), quant_type, int4 && block_size <= 0 ? 32 : block_size,
+                             s);
+    };
+    const bool widen =
+        k > 0 && scale_dtype == VM_HIP_DTYPE_F32 && widen_for_gemv(bf16, rows_m, k, n, int4, block_size);
+    if (k > 0 && !widen) {
+        const int rc = direct();
         if (rc != VM_HIP_EUNSUPPORTED) return rc;
     }
-    // Shapes the MFMA kernel does not take: half operands staged as fp32, [A |
-    // scales | C] in the per-stream buffer.
+    // Calls that the GEMV takes better and shapes the MFMA kernel does not take:
+    // half operands staged as fp32, [A | scales | C] in the per-stream buffer.
     const int64_t nblk = quant_type == VM_HIP_QUANT_INT4
                              ? (k + (block_size > 0 ? block_size : 32) - 1) / (block_size > 0 ? block_size : 32)
                              : (block_size > 0 ? (k + block_size - 1) / block_size : 1);
@@ -335,11 +356,21 @@ int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale, 
     const int64_t c_elems = rows_m * n;
     const auto align = [](int64_t e) { return (e + 63) & ~int64_t(63); };
     void* stage = nullptr;
-    VM_TRY(get_staging(s, static_cast<std::size_t>(align(a_elems) + align(s_elems) + align(c_elems)) * 4, &stage));
+    const std::size_t bytes = static_cast<std::size_t>(align(a_elems) + align(s_elems) + align(c_elems)) * 4;
+    int got = get_staging(s, bytes, &stage);
+    if (got != 0 && widen && scratch_refused(got)) {
+        const int rc = direct();
+        if (rc != VM_HIP_EUNSUPPORTED) return rc;
+        got = get_staging(s, bytes, &stage);
+    }
+    VM_TRY(got);
     float* a32 = static_cast<float*>(stage);
     float* s32 = a32 + align(a_elems);
     float* c32 = s32 + align(s_elems);
-    VM_TRY(vm_hip_half_to_f32(static_cast<const uint16_t*>(a), a_dtype, a32, a_elems, stream));
+    // The GEMV's INT4 sums carry 16 times the codes: bf16 activations, which
+    // reach fp32's end, go in divided by 16 (exact, subnormals too).
+    const bool shrink = widen && bf16 && int4;
+    VM_TRY(half_to_f32_times(static_cast<const uint16_t*>(a), bf16, a32, a_elems, shrink ? 0.0625f : 1.0f, s));
     const float* sc = static_cast<const float*>(scale);
     if (s_elems) {
         VM_TRY(vm_hip_half_to_f32(static_cast<const uint16_t*>(scale), scale_dtype, s32, s_elems, stream));
@@ -347,7 +378,7 @@ int vm_hip_qmm(const void* a, int a_dtype, const int8_t* wq, const void* scale, 
     }
     VM_TRY(qmm_f32_impl(a32, wq, sc, c32, rows_m, k, n, quant_type, block_size, s));
     hipLaunchKernelGGL(f32_to_half_kernel, dim3(blocks_for(c_elems, 256)), dim3(256), 0, s, c32,
-                       static_cast<uint16_t*>(c), c_elems, c_dtype == VM_HIP_DTYPE_BF16 ? 1 : 0);
+                       static_cast<uint16_t*>(c), c_elems, c_dtype == VM_HIP_DTYPE_BF16 ? 1 : 0, shrink ? 16.0f : 1.0f);
     return check_launch("QuantizedMatMul", s);
 }
 

@@ -305,7 +305,7 @@ __global__ void dequant_int4_kernel(const uint8_t* __restrict__ packed,
 
 // dtype.h:21-51 (exact widening, NaN made quiet) and :91-95.
 __global__ void half_to_f32_kernel(const uint16_t* __restrict__ src, float* __restrict__ dst,
-                                   int64_t count, int is_bf16) {
+                                   int64_t count, int is_bf16, float factor) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= count) return;
     const uint32_t h = src[i];
@@ -330,7 +330,7 @@ __global__ void half_to_f32_kernel(const uint16_t* __restrict__ src, float* __re
             f = sign | ((e + 112u) << 23) | (m << 13);
         }
     }
-    dst[i] = __uint_as_float(f);
+    dst[i] = factor == 1.0f ? __uint_as_float(f) : __uint_as_float(f) * factor;   // NaN bits stay at 1
 }
 
 unsigned grid_1d(int64_t count, int threads) {
@@ -338,6 +338,12 @@ unsigned grid_1d(int64_t count, int threads) {
 }
 
 }  // namespace
+int half_to_f32_times(const uint16_t* src, bool bf16, float* dst, int64_t count, float factor, hipStream_t stream) {
+    hipLaunchKernelGGL(half_to_f32_kernel, dim3(grid_1d(count, 256)), dim3(256), 0, stream, src, dst, count, bf16 ? 1 : 0,
+                       factor);
+    return check_launch("ConvertDtype", stream);
+}
+
 }  // namespace vmhip
 
 using namespace vmhip;
@@ -452,10 +458,7 @@ int vm_hip_half_to_f32(const uint16_t* src, int src_dtype, float* dst, int64_t c
     if (count < 0) return fail_inval("vm_hip_half_to_f32: negative count");
     if (count == 0) return 0;
     if (!src || !dst) return fail_inval("vm_hip_half_to_f32: null pointer");
-    auto s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(half_to_f32_kernel, dim3(grid_1d(count, 256)), dim3(256), 0, s, src, dst, count,
-                       src_dtype == VM_HIP_DTYPE_BF16 ? 1 : 0);
-    return check_launch("ConvertDtype", s);
+    return half_to_f32_times(src, src_dtype == VM_HIP_DTYPE_BF16, dst, count, 1.0f, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

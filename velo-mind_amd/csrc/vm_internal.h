@@ -91,6 +91,9 @@ private:
     FixedRegion* _previous;
 };
 
+// vm_hip_half_to_f32 times a power of two.
+int half_to_f32_times(const uint16_t* src, bool bf16, float* dst, int64_t count, float factor, hipStream_t stream);
+
 // Number of compute units of the current device (cached per device).
 int cu_count();
 
