@@ -54,6 +54,14 @@ def test_ragged_fp32(hip, kind, block, m, k, n):
     assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * mag + 1e-30)
 
 
+@pytest.mark.parametrize("kind,block", KINDS)
+@pytest.mark.parametrize("m,k,n", [(5, 1, 17), (33, 40, 130), (33, 41, 130), (6, 48, 31), (6, 49, 31), (6, 49, 100), (8, 72, 80),
+                                   (8, 73, 80), (900, 31, 151), (900, 31, 400)])
+def test_ragged_small(hip, kind, block, m, k, n):
+    # both sides of the sizes up to which a thread per output is the faster one
+    test_ragged_fp32(hip, kind, block, m, k, n)
+
+
 @pytest.mark.parametrize("kind,block", [("int8", 0), ("int8", 24), ("int4", 32), ("int4", 8)])
 @pytest.mark.parametrize("m", [1, 3])
 @pytest.mark.parametrize("k,n", [(31, 17), (64, 31), (576, 257), (2048, 515), (2048, 5633), (300, 26000 + 7), (5632, 2049)])
