@@ -38,7 +38,7 @@ def _inputs(batch, hq, hk, sq, sk, d, seed):
 
 
 @pytest.mark.parametrize("batch,hq,hk,sq,sk", [
-    (1, 2, 1, 5, 48), (1, 4, 4, 16, 64), (2, 4, 2, 17, 65), (1, 3, 1, 33, 127), (1, 5, 5, 64, 64), (2, 6, 3, 65, 129),
+    (1, 2, 1, 5, 48), (1, 3, 3, 7, 59), (1, 3, 3, 7, 60), (2, 10, 5, 48, 48), (1, 4, 4, 16, 64), (2, 4, 2, 17, 65), (1, 3, 1, 33, 127), (1, 5, 5, 64, 64), (2, 6, 3, 65, 129),
     (1, 2, 2, 100, 400),      # four key groups at head_dim 64
     (1, 8, 2, 31, 300),
     (3, 15, 5, 130, 130),     # two key groups

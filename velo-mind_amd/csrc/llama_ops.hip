@@ -583,10 +583,15 @@ namespace {
 hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
 
 // From here on attention runs on the matrix cores (head_dim 64 or 128): 512 x
-// 512, 15 heads of 64: 15.5 us against 117.6 with a wave per query row; 64 x 64,
-// 32 heads: 6.5 against 8.9; 5 x 700, 8 heads: 13.8 against 37.7.  With fewer
-// rows or keys there is nothing to gain (13 x 13, 16 heads of 128: 6 either way).
-constexpr int64_t kMfmaRows = 5, kMfmaKeys = 48;
+// 512, 15 heads of 64: 14.3 us against 114.6 with a wave per query row; 64 x 64,
+// 32 heads: 6.0 against 8.9; 5 x 700, 8 heads: 13.8 against 37.7.  With fewer
+// rows or keys there is nothing to gain (13 x 13, 16 heads of 128: 6 either way);
+// at head_dim 64 the chain of a wave per row is the shorter one below 60 keys
+// while the rows (of all heads) are few (16 x 48, 32 heads 5.4 us against 5.8, 33
+// x 56, 9 heads 5.6 against 5.9; 16 x 48, 64 heads 6.1 against 5.9).
+bool mfma_pays(int64_t rows, int64_t sq, int64_t sk, int64_t d) {
+    return sq >= 5 && sk >= 48 && (d != 64 || sk >= 60 || rows > 768);
+}
 
 constexpr size_t kChainMaxLds = 160 * 1024;   // dynamic LDS of the V-staging attention kernels (no static LDS)
 
@@ -840,7 +845,8 @@ int vm_hip_attention_f32(const float* q, const float* k, const float* v, float* 
     c.out_head = sq * d;
     c.scale = sc;
     c.causal = causal != 0;
-    if (sq >= kMfmaRows && sk >= kMfmaKeys && d == dv && attention_mfma_takes(c)) return attention_mfma(c, "FusedAttention", S(stream));
+    if (mfma_pays(rows, sq, sk, d) && d == dv && attention_mfma_takes(c))
+        return attention_mfma(c, "FusedAttention", S(stream));
     hipLaunchKernelGGL(attention_kernel, dim3(static_cast<unsigned>(rows)), dim3(64), static_cast<size_t>(lds),
                        S(stream), q, k, v, o, hq, hk, sq, sk, d, dv, sc, causal ? 1 : 0);
     return check_launch("FusedAttention", S(stream));
