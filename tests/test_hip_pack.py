@@ -53,10 +53,12 @@ def test_int4_bit_exact(hip, rows, cols, block):
     assert np.array_equal(s.view(np.uint32), s_ref.view(np.uint32))
 
 
-# Whole and partial 32-row groups, blocks that end inside a group of four,
-# 64 x 4-column workgroups with a remainder, and single-column loads (cols % 4).
+# Whole and partial 32-row groups, blocks that end inside a group of four, and
+# 64-column workgroups with a remainder; the last three fill the GPU with
+# workgroups of four columns a lane.
 @pytest.mark.parametrize("block", [32, 64, 128])
-@pytest.mark.parametrize("rows,cols", [(1, 4), (31, 260), (33, 256), (127, 1028), (129, 257), (300, 67), (2047, 515)])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (31, 260), (33, 256), (127, 1028), (129, 257), (300, 67), (2047, 515),
+                                       (33, 65540), (300, 21848), (2047, 4100)])
 def test_int4_row_held_blocks_bit_exact(hip, rows, cols, block):
     w = _normal(rows, cols, rows * 3 + cols + block)
     w[:, cols // 2] = 0.0

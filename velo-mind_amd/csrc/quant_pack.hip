@@ -409,10 +409,15 @@ int vm_hip_pack_int4(const float* w, uint8_t* packed, float* scale, int64_t rows
         const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(packed) % 4 == 0 && reinterpret_cast<uintptr_t>(scale) % 16 == 0;
         const int64_t groups = (rows + 127) / 128;   // (at most 65535, as the blocks above)
+        // Four columns a lane where that still leaves a workgroup for every
+        // compute unit; fewer are bound by one wave's 128 codes a lane and
+        // take one column (blocks of 32: 2048 x 4096, 256 workgroups, 10.2 us
+        // against 11.9 with one; 2048 x 2048 8.8 and 5.7, 512 x 1028 19.2 and 5.0).
+        const bool wide = vec && groups * ((cols + 255) / 256) >= 256;
 #define VM_PACK4(VX, GX)                                                                                             \
     hipLaunchKernelGGL((pack_int4_rows_kernel<VX, GX>), dim3(grid_1d(cols, 64 * VX), static_cast<unsigned>(groups)), \
                        dim3(256), 0, s, w, packed, scale, rows, cols)
-        if (vec) {
+        if (wide) {
             if (block == 32) VM_PACK4(4, 1);
             else if (block == 64) VM_PACK4(4, 2);
             else VM_PACK4(4, 4);
