@@ -31,8 +31,10 @@ def test_int4_kat_ties_and_nibbles(hip):
 
 @pytest.mark.parametrize("rows,cols", [(128, 256), (576, 1536), (33, 17), (1, 5), (7, 1),
                                        # two-pass path: ragged row chunks, columns past the last
-                                       # full workgroup, a single chunk, many chunks
-                                       (1000, 1028), (64, 260), (4099, 2048), (97, 4096)])
+                                       # full workgroup, a single chunk, many chunks, four columns a
+                                       # lane; the single pass's last row counts
+                                       (1000, 1028), (64, 260), (4099, 2048), (97, 4096), (108, 300), (109, 300),
+                                       (129, 513), (1000, 8196), (4099, 1028)])
 def test_int8_bit_exact(hip, rows, cols):
     w = ref_inputs.generate_random_weights(rows, cols, -1.5, 1.5)
     w[:, 0] = 0.0  # an all-zero column takes scale 1.0
@@ -70,7 +72,7 @@ def test_int4_row_held_blocks_bit_exact(hip, rows, cols, block):
 
 # The two-pass INT8 packer with single-column loads, row groups of 64 with a
 # remainder, and one chunk or the most.
-@pytest.mark.parametrize("rows,cols", [(64, 257), (65, 1001), (2049, 259), (4100, 301)])
+@pytest.mark.parametrize("rows,cols", [(109, 257), (129, 1001), (2049, 259), (4100, 301)])
 def test_int8_two_pass_odd_columns_bit_exact(hip, rows, cols):
     w = _normal(rows, cols, rows + cols)
     w[:, 3] = 0.0

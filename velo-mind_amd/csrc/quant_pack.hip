@@ -361,12 +361,18 @@ int vm_hip_pack_int8(const float* w, int8_t* q, float* scale, int64_t rows, int6
     // stream is not being captured (the row partials use the stream's
     // workspace, sized here; refused memory leaves the single pass, which
     // needs none) and the second pass's grid holds the rows.
-    const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
-                     reinterpret_cast<uintptr_t>(q) % 4 == 0;
+    // The single pass walks all rows of a column and is the faster one up to
+    // about 108 of them (64 x 2049 6.7 us against 9.4, 100 x 515 9.4 and 9.8, 128 x
+    // 515 11.4 and 9.9); four columns a lane pay from more than one workgroup of
+    // the second pass per compute unit (1000 x 8192 18.8 us against 24.8 with one
+    // column; 512 x 8192 12.9 and 12.6, 2048 x 2048 13.8 and 12.5, 512 x 516 17.6
+    // and 10.1).
     const int64_t row_groups = (rows + 4 * kPackRows - 1) / (4 * kPackRows);
+    const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(q) % 4 == 0 && row_groups * ((cols + 255) / 256) > 256;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (s) (void)hipStreamIsCapturing(s, &cap);
-    if (rows >= 64 && cols >= 256 && row_groups <= 65535 && cap == hipStreamCaptureStatusNone) {
+    if (rows > 108 && cols >= 256 && row_groups <= 65535 && cap == hipStreamCaptureStatusNone) {
         const int64_t col_groups = (cols + (vec ? 255 : 63)) / (vec ? 256 : 64);
         // about 1024 workgroups, whole steps of 64 rows each
         int64_t chunks = std::min<int64_t>({(1024 + col_groups - 1) / col_groups, row_groups, kPackMaxChunks});
