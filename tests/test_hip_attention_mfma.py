@@ -1,6 +1,7 @@
 """FusedAttention of several query rows on the matrix cores (head_dim 64 and
-128): edges of the 16-row query tiles and 64-key tiles, one, two and four key
-groups, grouped heads, batches, and values that a mask has to keep apart.
+128): edges of the 16-row query tiles and of the key blocks (32 keys, 16 at
+head_dim 128), two and four key groups, grouped heads, batches, values that a
+mask has to keep apart, and the sizes from which a wave per row takes the call.
 
 Bound: scores are fp32 dot products of d terms, |ds| <= d 2^-24 sum |q k|
 scale, which the exponential turns into a relative error of each weight; the
@@ -39,10 +40,10 @@ def _inputs(batch, hq, hk, sq, sk, d, seed):
 
 @pytest.mark.parametrize("batch,hq,hk,sq,sk", [
     (1, 2, 1, 5, 48), (1, 3, 3, 7, 59), (1, 3, 3, 7, 60), (2, 10, 5, 48, 48), (1, 4, 4, 16, 64), (2, 4, 2, 17, 65), (1, 3, 1, 33, 127), (1, 5, 5, 64, 64), (2, 6, 3, 65, 129),
-    (1, 2, 2, 100, 400),      # four key groups at head_dim 64
-    (1, 8, 2, 31, 300),
-    (3, 15, 5, 130, 130),     # two key groups
-    (2, 40, 8, 450, 450),     # more than 512 workgroups: one key group
+    (1, 2, 2, 100, 400), (1, 8, 2, 31, 300),
+    (3, 15, 5, 130, 130),     # 405 tiles of 16 rows: four key groups, as all above
+    (1, 64, 8, 150, 498),     # 640: two at head_dim 64
+    (2, 40, 8, 450, 450),     # 2320: two at either
 ])
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
@@ -55,19 +56,20 @@ def test_tiles(hip, batch, hq, hk, sq, sk, d, causal):
     assert np.all(np.abs(out - ref) <= bound), np.max(np.abs(out - ref) / bound)
 
 
+@pytest.mark.parametrize("hq,hk", [(2, 1), (416, 8)])   # four key groups, and two (2080 tiles of 16 rows)
 @pytest.mark.parametrize("d", [64, 128])
-def test_masked_values_do_not_reach_earlier_rows(hip, d):
+def test_masked_values_do_not_reach_earlier_rows(hip, d, hq, hk):
     # infinities and NaN in V and K at positions that some rows of a tile see
     # and others do not; a score of -inf beside finite ones; a row whose
     # every score is -inf (no softmax: NaN, as one row's kernel gives)
     sq = sk = 70
-    q, k, v = _inputs(1, 2, 1, sq, sk, d, d)
-    v[0, 0, 20, 3], v[0, 0, 21, 5], v[0, 0, 66, 0] = np.inf, np.nan, -np.inf
-    k[0, 0, 40, 7] = np.nan
-    k[0, 0, 50] = 0.0
-    k[0, 0, 50, 0] = np.inf
+    q, k, v = _inputs(1, hq, hk, sq, sk, d, d)
+    v[:, :, 20, 3], v[:, :, 21, 5], v[:, :, 66, 0] = np.inf, np.nan, -np.inf
+    k[:, :, 40, 7] = np.nan
+    k[:, :, 50] = 0.0
+    k[:, :, 50, 0] = np.inf
     q[..., 0] = -np.abs(q[..., 0])       # -inf scores at key 50
-    print(f"case attention masked specials d={d}", flush=True)
+    print(f"case attention masked specials d={d} hq={hq}", flush=True)
     out = hip.run_attention(q, k, v, 0.0, True)
     ref, bound = _reference(q, k, v, 1 / np.sqrt(d), True)
     finite = np.isfinite(ref)

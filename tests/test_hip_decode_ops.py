@@ -184,10 +184,10 @@ def test_rope_kv_append(hip):
     assert np.array_equal(dv.download(np.float32, vc.shape), vc)
 
 
-# (512, 0, ...) is TinyLlama's 512-token prefill (eight 64-key tiles for the
-# last query rows); (256, 300, ...) continues a cached prefix.  Grids of at
-# most 512 64-row tiles split each workgroup's keys over two wave pairs;
-# (600, 0, 64, ...) has 640 tiles and runs the one-group form.
+# (512, 0, ...) is TinyLlama's 512-token prefill (sixteen 32-key blocks for the
+# last query rows); (256, 300, ...) continues a cached prefix.  Up to 512 tiles
+# of 16 query rows (all heads) the four waves of a workgroup take four key
+# groups, beyond (TinyLlama's 1024, the 600-row calls' 2432) two.
 @pytest.mark.parametrize("rows,p0,heads,kv_heads,max_seq", [(19, 0, 8, 2, 96), (64, 0, 8, 2, 96), (70, 10, 8, 2, 96),
                                                         (200, 0, 32, 4, 256), (130, 77, 15, 5, 256),
                                                         (1, 40, 8, 8, 64), (512, 0, 32, 4, 768),

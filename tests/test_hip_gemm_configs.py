@@ -1,15 +1,13 @@
-"""Every MFMA GEMM tile variant (rows_m > 4), forced through the tuning
-overrides (VELOMIND_GEMM_CFG="BM,BN,S[,D]" for the small-tile kernel,
-VELOMIND_GEMM_WIDE="BM,BN,S,D,G" for the wide one), against the oracle.
+"""Every configuration of the MFMA GEMM (rows_m > 4, and 16-bit activations),
+forced through the tuning override VELOMIND_GEMM_WIDE="BM,BN,S,D": row tiles of
+16, 32 and (per-column INT8) 64, four waves or, with D = 2, eight, pairs of waves
+side by side in N with BN = 256, and S splits of K.
 
-Per-column INT8 takes either kernel; blockwise weights (INT4, INT8 with
-blocks) always take the wide kernel, which multiplies each 32-row chunk's
-fp32 sum by its block scale (codes exact in fp16), in its tile shapes with
-two 32 x 32 tiles per wave.  Covers K splits 1/2/4 (deterministic split-K
-reduction), partial M and N tiles, K ending half-way through a 64-row step,
-INT8 blocks of 32 and 96 rows, and block scales from 1e-7 to 1e3.  Bound:
-the north-star 1e-3 * max|ref|; test_activation_magnitudes also holds every
-kind to fp32 summation bounds against the reference loop.
+Per-column INT8, blockwise INT8 and INT4; fp32, fp16 and bf16; one split and
+three (deterministic split-K reduction), partial M and N tiles, every remainder
+of the pipelined loop, block scales from 1e-7 to 1e3.  Where the oracle is the
+reference the bound is 1e-3 * max|ref|; test_forced_config and
+test_activation_magnitudes hold every kind to fp32 summation bounds.
 """
 from __future__ import annotations
 
@@ -20,8 +18,6 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# (BM, BN) tile variants instantiated in velo-mind_amd/csrc/qmm_gemm.hip.
-TILES = [(16, 128), (32, 128), (64, 128), (128, 128), (16, 64), (32, 64), (64, 64)]
 TOL = 1e-3
 
 
@@ -45,43 +41,96 @@ def _weights(kind, k, n, rng, block):
     return q, s, 2, block
 
 
-@pytest.mark.parametrize("kind,block", [("int8", 0)])
-@pytest.mark.parametrize("bm,bn", TILES)
-def test_forced_tile(hip, monkeypatch, bm, bn, kind, block):
-    m, k, n = 40, 224, 336        # partial M and N tiles; 224 = 3.5 steps of 64
-    rng = np.random.default_rng(bm * 1000 + bn + block)
-    q, s, qt, blk = _weights(kind, k, n, rng, block)
-    oq = O.QUANT_INT4 if qt == 2 else O.QUANT_INT8
-    x = rng.standard_normal((m, k)).astype(np.float32)
-    ref = O.qmm(x, q.view(np.int8), s, k, oq, blk)
-    for splits in (1, 2, 4):
-        monkeypatch.setenv("VELOMIND_GEMM_CFG", f"{bm},{bn},{splits}")
-        print(f"case BM={bm} BN={bn} S={splits} kind={kind} block={block} m={m} k={k} n={n}", flush=True)
-        out = hip.run_qmm(x, q, s, k, qt, blk)
-        _check(out, ref)
-    monkeypatch.delenv("VELOMIND_GEMM_CFG")
+# (BM, BN, D) of the override -> row tile, 32-row tiles of it, waves, waves side
+# by side in N, and the loop's pipeline stages.
+CONFIGS = {
+    (16, 64, 1): (16, 1, 4, 1, 3), (16, 64, 2): (16, 1, 8, 1, 3), (32, 128, 1): (32, 1, 4, 1, 3), (32, 128, 2): (32, 1, 8, 1, 3),
+    (128, 128, 1): (32, 2, 4, 1, 4), (128, 256, 1): (32, 2, 4, 2, 4),   # per-column INT8
+    (32, 256, 1): (32, 1, 4, 2, 3),                                     # blockwise
+}
+KINDS = [("int8", 0), ("int8", 96), ("int4", 32), ("int4", 128)]
 
 
-@pytest.mark.parametrize("kind,block", [("int8", 0)])
-@pytest.mark.parametrize("bm,deep", [(16, 4), (16, 8), (32, 4), (32, 8)])
-@pytest.mark.parametrize("m", [5, 16, 40])
-def test_forced_deep(hip, monkeypatch, bm, deep, kind, block, m):
-    # K = 992 rows = 15.5 steps of 64: with D steps in flight the split
-    # count is at least ceil(16 / D), and the last split is partial (its
-    # trailing steps read zeros); N = 336 leaves a partial column tile.
-    k, n = 992, 336
-    rng = np.random.default_rng(bm * 100 + deep * 10 + m + block)
-    q, s, qt, blk = _weights(kind, k, n, rng, block)
-    oq = O.QUANT_INT4 if qt == 2 else O.QUANT_INT8
-    x = rng.standard_normal((m, k)).astype(np.float32)
-    ref = O.qmm(x, q.view(np.int8), s, k, oq, blk)
-    steps = (k + 63) // 64
-    for splits in sorted({-(-steps // deep), -(-steps // deep) + 1, 16}):
-        monkeypatch.setenv("VELOMIND_GEMM_CFG", f"{bm},64,{splits},{deep}")
-        print(f"case BM={bm} D={deep} S={splits} kind={kind} block={block} m={m} k={k} n={n}", flush=True)
-        out = hip.run_qmm(x, q, s, k, qt, blk)
-        _check(out, ref)
-    monkeypatch.delenv("VELOMIND_GEMM_CFG")
+def _configs(kind, block, pieces=True):
+    for cfg, (tile, mt, _, nw, _) in CONFIGS.items():
+        if (mt == 1 or block == 0) and (nw == 1 or mt == 2 or block > 0) and (pieces or (mt == 1 and nw == 1)):
+            yield cfg
+
+
+def _forced_k(kind, block, cfg, splits, turns):
+    """K for which every wave but the last runs `turns` chunks and the number
+    of splits is the one asked for; the launcher's arithmetic, checked."""
+    tile, _, waves, nw, _ = CONFIGS[cfg]
+    chunk = 16 if block == 0 and tile == 32 else 32
+    units = splits * (waves // nw)
+    chunks = units * turns - 1
+    per_wave = -(-chunks // units)
+    assert per_wave == turns and -(-chunks // (per_wave * (waves // nw))) == splits
+    return chunk * chunks
+
+
+def _random_weights(rng, kind, block, k, n):
+    """(codes, scales, dense weights in 64 bits, quant type)"""
+    nb = -(-k // block) if block else 1
+    s = (rng.random((nb, n)) * 0.01 + 1e-4).astype(np.float32)
+    if kind == "int8":
+        q = rng.integers(-127, 128, (k, n), dtype=np.int8)
+        v = q
+    else:
+        q = rng.integers(0, 256, ((k + 1) // 2, n)).astype(np.uint8)
+        v = np.empty((2 * q.shape[0], n), np.int8)
+        v[0::2], v[1::2] = (q.view(np.int8) << 4) >> 4, q.view(np.int8) >> 4
+        v = v[:k]
+    return q, s, v.astype(np.float64) * s.astype(np.float64).repeat(block or k, 0)[:k], 2 if kind == "int4" else 1
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("kind,block,cfg", [(*kb, c) for kb in KINDS for c in _configs(*kb)])
+def test_forced_config(hip, monkeypatch, kind, block, cfg, splits):
+    m, n = 150, 531   # partial tiles of every width, a last quad that moves back
+    stages = CONFIGS[cfg][4]
+    for turns in range(stages + 1, 2 * stages + 1):   # the loop runs, then every remainder
+        k = _forced_k(kind, block, cfg, splits, turns)
+        rng = np.random.default_rng(k + cfg[0] + cfg[1] + splits)
+        q, s, wd, qt = _random_weights(rng, kind, block, k, n)
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        monkeypatch.setenv("VELOMIND_GEMM_WIDE", "%d,%d,%d,%d" % (cfg[0], cfg[1], splits, cfg[2]))
+        print(f"case forced {kind} block={block} {cfg} S={splits} turns={turns} m={m} k={k} n={n}", flush=True)
+        out = hip.run_qmm(x, q, s, k, qt, block).astype(np.float64)
+        bound = (2.0 ** -22 + 2 * k * 2.0 ** -24) * 1.01 * (np.abs(x.astype(np.float64)) @ np.abs(wd))
+        assert np.all(np.abs(out - x.astype(np.float64) @ wd) <= bound)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("half_scale", [False, True])
+@pytest.mark.parametrize("m", [100, 150])   # rows as they lie, and staged in operand order
+@pytest.mark.parametrize("kind,block", KINDS)
+def test_forced_config_half(hip, monkeypatch, kind, block, m, half_scale, bf16):
+    n = 531
+    for cfg in _configs(kind, block, pieces=m > 128):
+        for splits in (1, 3):
+            k = _forced_k(kind, block, cfg, splits, CONFIGS[cfg][4] + 2)
+            k -= k % 32 if m <= 128 else 0   # (rows are read as they lie in whole chunks only)
+            rng = np.random.default_rng(k + cfg[0] + cfg[1] + m)
+            q, s, wd, qt = _random_weights(rng, kind, block, k, n)
+            wide = (lambda b: (b.astype(np.uint32) << 16).view(np.float32)) if bf16 else (
+                lambda b: b.view(np.float16).astype(np.float32))
+            bits = O.f32_to_bf16_bits if bf16 else O.f32_to_f16_bits
+            a, sb = bits(rng.standard_normal((m, k)).astype(np.float32)), bits(s)
+            if half_scale:
+                wd *= (wide(sb).astype(np.float64) / s).repeat(block or k, 0)[:k]
+            dt = hip.DTYPE_BF16 if bf16 else hip.DTYPE_F16
+            da, dq, ds, dc = (hip.DeviceBuffer.from_array(t) for t in (a, q.view(np.int8), sb if half_scale else s,
+                                                                       np.zeros((m, n), np.uint16)))
+            monkeypatch.setenv("VELOMIND_GEMM_WIDE", "%d,%d,%d,%d" % (cfg[0], cfg[1], splits, cfg[2]))
+            print(f"case forced half bf16={bf16} {kind} block={block} {cfg} S={splits} m={m} k={k} n={n}", flush=True)
+            hip.qmm(da.addr, dt, dq.addr, ds.addr, dt if half_scale else hip.DTYPE_F32, dc.addr, dt, m, k, n, qt, block)
+            out = wide(dc.download(np.uint16, (m, n))).astype(np.float64)
+            aw = wide(a).astype(np.float64)
+            ref = aw @ wd
+            bound = (2.0 ** -8 if bf16 else 2.0 ** -11) * 1.01 * np.abs(ref) + 2 * k * 2.0 ** -24 * (
+                np.abs(aw) @ np.abs(wd)) + 2.0 ** -24
+            assert np.all(np.abs(out - ref) <= bound), (cfg, splits)
 
 
 @pytest.mark.parametrize("mag", [1e-7, 1e-3, 1e3])
@@ -116,7 +165,7 @@ def test_split_k_deterministic(hip, monkeypatch):
     rng = np.random.default_rng(5)
     q, s = O.quantize_int4((rng.standard_normal((k, n)) * 0.02).astype(np.float32), 32)
     x = rng.standard_normal((m, k)).astype(np.float32)
-    monkeypatch.setenv("VELOMIND_GEMM_WIDE", "64,128,8,2,1")   # eight K splits of the blockwise kernel
+    monkeypatch.setenv("VELOMIND_GEMM_WIDE", "32,128,8,2")   # eight K splits, eight waves
     outs = [hip.run_qmm(x, q, s, k, hip.QUANT_INT4, 32) for _ in range(3)]
     for o in outs[1:]:
         assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32))
@@ -136,7 +185,7 @@ def _magnitude_rows(rng, k):
 
 
 @pytest.mark.parametrize("kind,block", [("int8", 0), ("int8_block", 32), ("int4", 32)])
-@pytest.mark.parametrize("reps", [1, 8, 30])      # m = 6, 48, 180: DEEP, small-M and large-M tiles
+@pytest.mark.parametrize("reps", [1, 8, 30])      # m = 6, 48, 180: 16- and 32-row tiles
 def test_activation_magnitudes(hip, kind, block, reps):
     import llama_oracle as LO
 
@@ -167,57 +216,21 @@ def test_activation_magnitudes(hip, kind, block, reps):
     assert np.all(np.abs(out - ref) <= bound), f"worst ratio {np.max(np.abs(out - ref) / bound):.3e}"
 
 
-# Wide-tile variants, forced through VELOMIND_GEMM_WIDE="BM,BN,S,D,G": per-column
-# INT8 takes all of them, blockwise weights the ones with two 32 x 32 tiles per wave.
-WIDE_INT8 = [(128, 128, 2, 1), (128, 128, 2, 2), (128, 128, 4, 1), (64, 128, 2, 1), (64, 128, 4, 1), (128, 64, 2, 1),
-             (128, 64, 2, 2), (64, 256, 2, 1)]
-WIDE_BLOCK = [(128, 64, 2, 1), (128, 64, 2, 2), (64, 128, 2, 1)]
-WIDE_CASES = ([("int8", 0) + t for t in WIDE_INT8] +
-              [kb + t for kb in (("int8_block", 32), ("int8_block", 96), ("int4", 32), ("int4", 64)) for t in WIDE_BLOCK])
-
-
-@pytest.mark.parametrize("kind,block,bm,bn,depth,groups", WIDE_CASES)
-@pytest.mark.parametrize("m", [6, 40, 130])
-def test_forced_wide(hip, monkeypatch, bm, bn, depth, groups, kind, block, m):
-    # K = 224 = 3.5 steps of 64; N = 336 leaves partial tiles for every BN;
-    # m = 130 leaves a 2-row M tile after 128.
-    k, n = 224, 336
-    rng = np.random.default_rng(bm * 7 + bn + depth * 3 + groups * 5 + block + m)
-    q, s, qt, blk = _weights(kind, k, n, rng, block)
-    oq = O.QUANT_INT4 if qt == 2 else O.QUANT_INT8
-    x = rng.standard_normal((m, k)).astype(np.float32)
-    ref = O.qmm(x, q.view(np.int8), s, k, oq, blk)
-    for splits in (1, 2, 4):
-        monkeypatch.setenv("VELOMIND_GEMM_WIDE", f"{bm},{bn},{splits},{depth},{groups}")
-        print(f"case wide BM={bm} BN={bn} D={depth} G={groups} S={splits} kind={kind} block={block} m={m} k={k} n={n}",
-              flush=True)
-        out = hip.run_qmm(x, q, s, k, qt, blk)
-        _check(out, ref)
-    monkeypatch.delenv("VELOMIND_GEMM_WIDE")
-
-
 @pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
-def test_wide_long_k(hip, monkeypatch, kind, block):
-    # K = 2048: every ring stage wraps several times; the default rule's splits
+def test_long_k(hip, kind, block):
+    # K = 2048: the default rule's splits, every stage used several times
     m, k, n = 200, 2048, 512
     rng = np.random.default_rng(91 + block)
     q, s, qt, blk = _weights(kind, k, n, rng, block)
-    oq = O.QUANT_INT4 if qt == 2 else O.QUANT_INT8
     x = rng.standard_normal((m, k)).astype(np.float32)
-    ref = O.qmm(x, q.view(np.int8), s, k, oq, blk)
-    print(f"case wide long-k default kind={kind} m={m} k={k} n={n}", flush=True)
-    _check(hip.run_qmm(x, q, s, k, qt, blk), ref)
-    forced = "128,128,3,2,2" if kind == "int8" else "128,64,3,2,2"
-    monkeypatch.setenv("VELOMIND_GEMM_WIDE", forced)
-    print(f"case wide long-k {forced} kind={kind}", flush=True)
-    _check(hip.run_qmm(x, q, s, k, qt, blk), ref)
-    monkeypatch.delenv("VELOMIND_GEMM_WIDE")
+    print(f"case long k kind={kind} m={m} k={k} n={n}", flush=True)
+    _check(hip.run_qmm(x, q, s, k, qt, blk), O.qmm(x, q.view(np.int8), s, k, O.QUANT_INT4 if qt == 2 else O.QUANT_INT8, blk))
 
 
 @pytest.mark.parametrize("kind,block", [("int8", 0), ("int4", 32)])
 @pytest.mark.parametrize("m,n", [(384, 300), (401, 4500), (700, 1100), (1025, 2600)])
 def test_row_panels(hip, kind, block, m, n):
-    # tiles are numbered in panels of about 256 rows, the last one shorter:
+    # past 384 rows tiles are numbered in panels of rows, the last one shorter:
     # every tile of every panel is written
     k = 96
     rng = np.random.default_rng(m + n)

@@ -101,7 +101,7 @@ def test_config3_prefill(hip, m, qt):
 
 @pytest.mark.parametrize("qt", ["int4", "int8"])
 def test_output_of_more_than_2gib(hip, qt):
-    """A 4100 x 131072 fp32 output (2.05 GiB) on the wide MFMA kernel, which
+    """A 4100 x 131072 fp32 output (2.05 GiB) on the MFMA kernel, which
     addresses C from a 64-bit base per 128-row tile: rows on both sides of
     the 2 GiB mark match the reference loop."""
     m, k, n = 4100, 32, 131072
@@ -260,8 +260,9 @@ def test_graph_keeps_workspace_after_growth(hip):
     g.begin()
     hip.qmm_f32(da.addr, dp.addr, ds.addr, d_graph.addr, 1, k, n, hip.QUANT_INT4, 32, st)
     g.end()
-    # The two-pass INT8 pack of a 2048 x 8192 matrix keeps 64 x 8192 row
-    # partials in the same workspace: more than the GEMV sized it for.
+    # The two-pass INT8 pack of a 2048 x 8192 matrix keeps up to 32 x 8192
+    # partial column maxima in the same workspace: more than the GEMV sized it
+    # for.
     rows, cols = 2048, 8192
     w = _normal((rows, cols), 83, 0.02)
     dw = hip.DeviceBuffer.from_array(w)

@@ -2,8 +2,8 @@
 (vm_hip_add_rmsnorm_stage_f32, vm_hip_silu_mul_stage_f32,
 vm_hip_qmm_staged_f32): the GEMM on the staged buffer equals
 vm_hip_qmm_f32 on the fp32 rows the producer also writes, bit for bit, in
-both layouts (row-major for the small-tile kernel, operand order for the
-wide kernel) and for INT8 per column, INT8 blockwise and INT4; the fp32
+both layouts (row-major for few rows of per-column INT8, else the MFMA
+kernel's operand order) and for INT8 per column, INT8 blockwise and INT4; the fp32
 rows equal the plain producers' (SiLU exactly, RMSNorm to the rounding of
 its sum of squares); the oracle bounds the result as for every GEMM."""
 from __future__ import annotations
@@ -51,7 +51,7 @@ def _gemm_both(H, lib, staged, a32, q, s, rows, k, n, qt, blk, layout):
 @pytest.mark.parametrize("kind", ["int8", "int8_block", "int4"])
 def test_add_rmsnorm_stage(hip, rows, n, want, kind):
     if kind != "int8":
-        want = A_PIECES   # blockwise scales always take the wide kernel's operand order
+        want = A_PIECES   # blockwise scales: always operand order
     H, lib = hip, hip.open_library()
     k = 2048
     rng = np.random.default_rng(rows + n + len(kind))
@@ -81,7 +81,7 @@ def test_add_rmsnorm_stage(hip, rows, n, want, kind):
 @pytest.mark.parametrize("kind", ["int8", "int4"])
 def test_silu_mul_stage(hip, rows, inter, n, want, kind):
     if kind != "int8":
-        want = A_PIECES   # blockwise scales always take the wide kernel's operand order
+        want = A_PIECES   # blockwise scales: always operand order
     H, lib = hip, hip.open_library()
     rng = np.random.default_rng(rows + inter + len(kind))
     gu = rng.standard_normal((rows, 2 * inter)).astype(np.float32) * 3
@@ -126,7 +126,7 @@ def test_stage_rows_with_extreme_magnitudes(hip):
 def test_stage_arguments(hip):
     H, lib = hip, hip.open_library()
     assert _layout(lib, 4, 2048, 2048, 2, 32)[0] == A_FP32     # GEMV rows take fp32 A
-    assert _layout(lib, 64, 2040, 2048, 2, 32)[0] == A_FP32    # K % 32 != 0: the generic kernel
+    assert _layout(lib, 64, 2040, 2048, 2, 32)[0] == A_FP32    # K % 32 != 0: staged by the GEMM itself
     buf = H.DeviceBuffer(1 << 20)
     x = H.DeviceBuffer(64 * 2048 * 4)
     assert lib.vm_hip_silu_mul_stage_f32(x.ptr, buf.ptr, 7, None, 8, 1024, None) == H.EINVAL

@@ -17,21 +17,20 @@ def _layout(rows, k, n, qt=H.QUANT_INT4, blk=32):
     return lay.value, nbytes.value
 
 
-def test_wide_kernel_taken_at_prefill_shapes():
-    # TinyLlama's gate|up at a 512-token prompt: the wide kernel's operand order.
+def test_operand_order_at_prefill_shapes():
+    # TinyLlama's gate|up at a 512-token prompt.
     assert _layout(512, 2048, 5632)[0] == H.A_PIECES
     assert _layout(512, 2048, 5632, H.QUANT_INT8, 0)[0] == H.A_PIECES
 
 
-def test_blockwise_weights_always_take_the_wide_kernel():
-    # Only the wide kernel applies block scales to each chunk's fp32 sum;
-    # it addresses C from a 64-bit base per 128-row tile, so outputs of
-    # 2 GiB and more stay on it too (tests/test_hip_qmm.py writes one).
+def test_blockwise_weights_always_take_operand_order():
+    # C is addressed with 64 bits, so outputs of 2 GiB and more are staged
+    # too (tests/test_hip_qmm.py writes one).
     for rows in (5, 16, 64, 512, 4096):
         assert _layout(rows, 2048, 5632)[0] == H.A_PIECES
     assert _layout(4096, 2048, 131072)[0] == H.A_PIECES
     assert _layout(16, 2048, 5632, H.QUANT_INT8, 32)[0] == H.A_PIECES
-    # per-column INT8 keeps the small-tile kernel for few rows
+    # few rows of per-column INT8: row-major
     assert _layout(16, 2048, 5632, H.QUANT_INT8, 0)[0] == H.A_ROWS
 
 

@@ -89,8 +89,8 @@ def test_noalloc_on_a_stream_then_null_stream(hip):
 
 
 def test_noalloc_refuses_scratch_beyond_its_array(hip, monkeypatch):
-    # 130 rows INT4 at K=4096 forced to sixteen K splits of the wide kernel
-    # (the tuning override) take 16 x 130 x 8192 fp32 partials (65 MiB),
+    # 130 rows INT4 at K=4096 forced to sixteen K splits (the tuning
+    # override) take 16 x 130 x 8192 fp32 partials (65 MiB),
     # more than the 14 MiB the static array holds.
     m, k, n = 130, 4096, 8192
     da = hip.DeviceBuffer(m * k * 4)
