@@ -29,7 +29,7 @@ ARCH = "gfx950"
 
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
-    # Packed-FP32 VALU forms stay disabled on this pool.
+    # No packed-FP32 VALU forms: some have given wrong results now and then.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # Bit-exact packing needs IEEE division and no fast-math rewriting.
     "-fhip-fp32-correctly-rounded-divide-sqrt", "-fno-fast-math",

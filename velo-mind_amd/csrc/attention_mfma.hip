@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_mfma_kernel(const Atten
     // Tiles in descending order of the keys they see; of a grid that fits the
     // GPU two workgroups to a compute unit, the second one per unit comes in
     // ascending order, so that a unit's two together see about as many as any
-    // other's (512 cached rows, 32 heads: 26.2 -> 22.7 us).
+    // other's (512 cached rows, 32 heads: 24.6 -> 20.8 us).
     int order = static_cast<int>(blockIdx.x);
     if (fold > 0 && order >= fold) order = fold + static_cast<int>(gridDim.x) - 1 - order;
     const int bh = order % bh_count;
@@ -337,11 +337,12 @@ int launch(const AttentionCall& c, const char* op, hipStream_t stream) {
 // last rows' chain of blocks the most, while the 16-row tiles are few enough
 // that chains and not throughput bound the call, else two (sharing K and V
 // lines in L1 between two row blocks).  MI355X: 512 x 512, 15 heads of 64 (480
-// tiles) 15.5 us against 18.4 with two, 16 x 2000, 8 heads 29 against 53; 512
-// cached rows, 32 heads of 64 (1024 tiles) 27.7 against 22.7, 1500 rows 123
-// against 120; 150 x 498, 128 heads of 128 (1280 tiles) 71 against 84, 1000 x
-// 1500, 64 heads (4032 tiles) 389 against 380.  One group was slower
-// everywhere but on a few keys.
+// tiles) 14.4 us against 17.1 with two, 16 x 2000, 8 heads 28.7 against 52.8; 512
+// cached rows, 32 heads of 64 (1024 tiles) 25.5 against 20.7, 1500 rows 122
+// against 116; 150 x 498, 128 heads of 128 (1280 tiles) 68 against 81, 1000 x
+// 1500, 64 heads (4032 tiles) 386 against 378.  One group (64 rows a
+// workgroup, nothing to merge) is faster for 128 cached heads of 64 (700 rows
+// 103 against 112) and slower below (512 rows, 48 heads 37.6 against 33.1).
 int key_groups(const AttentionCall& c) {
     const int64_t tiles = (static_cast<int64_t>(c.rows) + 15) / 16 * c.batch * c.heads;
     return tiles <= (c.head_dim == 64 ? 512 : 2048) ? 4 : 2;

@@ -584,7 +584,7 @@ hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
 
 // From here on attention runs on the matrix cores (head_dim 64 or 128): 512 x
 // 512, 15 heads of 64: 14.3 us against 114.6 with a wave per query row; 64 x 64,
-// 32 heads: 6.0 against 8.9; 5 x 700, 8 heads: 13.8 against 37.7.  With fewer
+// 32 heads: 5.8 against 8.9; 5 x 700, 8 heads: 13.8 against 37.7.  With fewer
 // rows or keys there is nothing to gain (13 x 13, 16 heads of 128: 6 either way);
 // at head_dim 64 the chain of a wave per row is the shorter one below 60 keys
 // while the rows (of all heads) are few (16 x 48, 32 heads 5.4 us against 5.8, 33

@@ -471,6 +471,7 @@ void qmm_quad_kernel(const QuadArgs g) {
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    static_assert(D == 3 || D == 4, "the loop below");
     // D - 1 stages in flight ahead of the one in use
 #pragma unroll
     for (int d = 0; d + 1 < D; ++d) load(st[d]);
@@ -482,7 +483,6 @@ void qmm_quad_kernel(const QuadArgs g) {
         step(integral_constant<int, 1>{}, kRefill);
         if constexpr (D > 2) step(integral_constant<int, 2 % D>{}, kRefill);
         if constexpr (D > 3) step(integral_constant<int, 3 % D>{}, kRefill);
-        if constexpr (D > 4) step(integral_constant<int, 4 % D>{}, kRefill);
     }
     constexpr integral_constant<bool, false> kLast{};
     if (left > 0) step(integral_constant<int, 0>{}, kLast);
@@ -490,8 +490,6 @@ void qmm_quad_kernel(const QuadArgs g) {
         if (left > 1) step(integral_constant<int, 1>{}, kLast);
     if constexpr (D > 3)
         if (left > 2) step(integral_constant<int, 2 % D>{}, kLast);
-    if constexpr (D > 4)
-        if (left > 3) step(integral_constant<int, 3 % D>{}, kLast);
 
     // ---- epilogue
     auto column_scale = [&]() {
@@ -784,8 +782,9 @@ struct QuadConfig {
 // choose alike; it refuses longer A, and takes no 16-bit calls, and these have
 // all their splits (M = 512, 8192 x 512 INT8 33.6 us in four splits, 44.5 in one).
 // VELOMIND_GEMM_WIDE="BM,BN,S,D[,G]" or VELOMIND_GEMM_CFG="BM,BN,S[,D]" force
-// the row tile (nearest to BM), paired waves with BN of 256 or more, S splits
-// and, with D or G of 2, eight waves.
+// the row tile (16 up to BM = 16, per-column INT8 64 from BM = 128, else 32),
+// paired waves with BN of 256 or more (64-row tiles and blockwise kinds), S
+// splits and, with D or G of 2, eight waves (not 64-row tiles).
 template <int KIND, int AM, int EL>
 QuadConfig choose_quad(int m, int k, int n, std::size_t a_bytes) {
     const double code_bytes = (KIND == 2 ? 0.5 : 1.0) * k * n;
