@@ -255,9 +255,12 @@ void qmm_quad_kernel(const QuadArgs g) {
     }
     const int split = lin / (g.tiles_n * g.tiles_m);
     const int in_split = lin - split * g.tiles_n * g.tiles_m;
-    const int panel = in_split / (g.panel * g.tiles_n);
-    const int in_panel = in_split - panel * g.panel * g.tiles_n;
-    const int panel_rows = min(g.panel, g.tiles_m - panel * g.panel);
+    int panel = 0, in_panel = in_split, panel_rows = g.tiles_m;
+    if (EL == EL_F32 && g.panel < g.tiles_m) {   // (16-bit A: one panel)
+        panel = in_split / (g.panel * g.tiles_n);
+        in_panel = in_split - panel * g.panel * g.tiles_n;
+        panel_rows = min(g.panel, g.tiles_m - panel * g.panel);
+    }
     const int tile_x = in_panel / panel_rows;
     const int tile_y = panel * g.panel + in_panel - tile_x * panel_rows;
     const int splits = static_cast<int>(gridDim.x) / (g.tiles_n * g.tiles_m);
