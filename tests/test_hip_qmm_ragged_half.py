@@ -55,8 +55,8 @@ def test_ragged_fp32(hip, kind, block, m, k, n):
 
 
 @pytest.mark.parametrize("kind,block", KINDS)
-@pytest.mark.parametrize("m,k,n", [(5, 1, 17), (33, 40, 130), (33, 41, 130), (6, 48, 31), (6, 49, 31), (6, 49, 100), (8, 72, 80),
-                                   (8, 73, 80), (900, 31, 151), (900, 31, 400)])
+@pytest.mark.parametrize("m,k,n", [(5, 1, 17), (33, 40, 130), (33, 46, 40), (33, 46, 41), (6, 48, 31), (6, 80, 40), (6, 49, 100), (8, 72, 80),
+                                   (8, 73, 80), (900, 31, 151), (900, 31, 480)])
 def test_ragged_small(hip, kind, block, m, k, n):
     # both sides of the sizes up to which a thread per output is the faster one
     test_ragged_fp32(hip, kind, block, m, k, n)

@@ -303,13 +303,14 @@ int gemm_qmm_staged_f32(const GemmPlan& plan, const _Float16* ah, const int* row
 // Ragged calls so small that one launch with a thread per output, a serial
 // chain over K, takes less than staging and GEMM, which take 7 to 8 us at any
 // such size (generic / MFMA): per-column INT8 33 rows of 31 x 130 4.7 / 7.3 us,
-// of 48 x 1027 6.4 / 7.7, of 63 x 130 7.7 / 7.7, of 63 x 65 6.6 / 7.4, 512 rows of
-// 31 x 515 5.2 / 8.7, of 31 x 1027 8.1 / 8.1; INT4 33 rows of 33 x 130 6.4 / 8.1, of
-// 48 x 130 8.4 / 7.9, 512 rows of 16 x 515 6.0 / 8.4, of 31 x 515 8.9 / 8.3.
+// of 48 x 1027 6.4 / 7.7, of 63 x 130 7.7 / 7.7, of 63 x 65 6.6 / 7.4, of 80 x 31
+// 7.1 / 7.7, 512 rows of 48 x 515 6.8 / 7.7, of 31 x 1027 8.1 / 8.1; INT4 33 rows
+// of 33 x 130 6.4 / 8.1, of 45 x 17 7.2 / 7.9, of 48 x 130 8.4 / 7.9, 512 rows of
+// 16 x 515 5.9 / 8.4, of 31 x 515 8.9 / 8.3.
 static bool generic_is_faster(int kind, int m, int k, int n) {
     const double work = static_cast<double>(m) * n * k;
-    if (kind == 0) return work <= 10e6 && (k <= 48 || (k <= 72 && n <= 80));
-    return work <= 4.2e6 && k <= 40;
+    if (kind == 0) return work <= 13e6 && (k <= 48 || (k <= 72 && n <= 80) || (k <= 80 && n <= 40));
+    return work <= 4.4e6 && (k <= 40 || (k <= 46 && n <= 40));
 }
 
 int gemm_qmm_f32(const float* a, const uint8_t* wq, const float* scale, float* c, int m, int k, int n,
